@@ -82,19 +82,18 @@ __device__ __forceinline__ void solve_stage(char* lds, const canary_batch_solve&
         sv.vmapM, sv.vmapP, sv.elemtobndy, rka, rkb, sv.dt, p, sv.advection);
 }
 
-// One workgroup per work-table entry; workgroup b takes entry
-// (b & 7) * chunk + (b >> 3) (grid = 8 * chunk), so XCD b & 7 gets a
-// contiguous run of the table.  (A grid-stride loop over entries keeps the
+// One workgroup per work-table entry, in the block order of stage_block (grid =
+// 8 * order.chunk): runs of the table dealt to the XCDs.  (A grid-stride loop over entries keeps the
 // per-thread face and LDS addressing live across iterations and costs
 // about 100 VGPRs in 3D; one entry per workgroup does not.)
 template <class Phys, int NQ, int EPW, bool PREP>
 __global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT)) void batched_kernel(
     const canary_batch_solve* __restrict__ solves, const canary_batch_item* __restrict__ items,
-    int64_t nitems, int64_t chunk, int parity, double rka, double rkb,
+    int64_t nitems, BlockOrder order, int parity, double rka, double rkb,
     const crpow::KappaTable* __restrict__ ktabs, int nktab) {
   using C = FusedCfg<Phys, NQ, EPW, false>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
-  const int64_t w = stage_block(blockIdx.x, chunk, parity);  // direction alternates per stage
+  const int64_t w = stage_block(blockIdx.x, order);  // direction alternates per stage
   if (w >= nitems) return;
   const canary_batch_item it = items[w];
   const canary_batch_solve& sv = solves[it.solve];
@@ -160,10 +159,10 @@ __device__ __forceinline__ void all_item(char* lds, const canary_batch_solve& sv
 template <class Phys, bool PREP>
 __global__ __launch_bounds__(MAXT) void batched_all_kernel(
     const canary_batch_solve* __restrict__ solves, const canary_batch_item* __restrict__ items,
-    int64_t nitems, int64_t chunk, int parity, double rka, double rkb,
+    int64_t nitems, BlockOrder order, int parity, double rka, double rkb,
     const crpow::KappaTable* __restrict__ ktabs, int nktab) {
   __shared__ __attribute__((aligned(16))) char lds[all_lds<Phys>()];
-  const int64_t w = stage_block(blockIdx.x, chunk, parity);
+  const int64_t w = stage_block(blockIdx.x, order);
   if (w >= nitems) return;
   const canary_batch_item it = items[w];
   const canary_batch_solve& sv = solves[it.solve];
@@ -206,12 +205,12 @@ __global__ __launch_bounds__(MAXT) void batched_all_kernel(
 template <class Phys, bool PREP>
 int run_all(const canary_batch_solve* solves, const canary_batch_item* items, int64_t nitems,
             int parity, double rka, double rkb, hipStream_t st) {
-  const int64_t chunk = (nitems + 7) / 8;
-  if (chunk > ((int64_t)1 << 27)) return CANARY_ERR_ARG;
+  if (nitems > ((int64_t)1 << 30)) return CANARY_ERR_ARG;
+  const BlockOrder order = block_order(nitems, parity);
   int nktab = 0;
   const crpow::KappaTable* ktabs = Phys::HAS_P ? kappa_tables(&nktab) : nullptr;
-  batched_all_kernel<Phys, PREP><<<dim3((unsigned)(8 * chunk)), dim3(MAXT), 0, st>>>(
-      solves, items, nitems, chunk, parity, rka, rkb, ktabs, nktab);
+  batched_all_kernel<Phys, PREP><<<dim3((unsigned)(8 * order.chunk)), dim3(MAXT), 0, st>>>(
+      solves, items, nitems, order, parity, rka, rkb, ktabs, nktab);
   return hipGetLastError() == hipSuccess ? 0 : CANARY_ERR_LAUNCH;
 }
 
@@ -229,12 +228,12 @@ int run_which(int* epw, int* threads, const canary_batch_solve* solves,
       *threads = NT;
       return 0;
     }
-    const int64_t chunk = (nitems + 7) / 8;
-    if (chunk > ((int64_t)1 << 27)) return CANARY_ERR_ARG;
+    if (nitems > ((int64_t)1 << 30)) return CANARY_ERR_ARG;
+    const BlockOrder order = block_order(nitems, parity);
     int nktab = 0;
     const crpow::KappaTable* ktabs = Phys::HAS_P ? kappa_tables(&nktab) : nullptr;
-    batched_kernel<Phys, NQ, E, PREP><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, st>>>(
-        solves, items, nitems, chunk, parity, rka, rkb, ktabs, nktab);
+    batched_kernel<Phys, NQ, E, PREP><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, st>>>(
+        solves, items, nitems, order, parity, rka, rkb, ktabs, nktab);
     return hipGetLastError() == hipSuccess ? 0 : CANARY_ERR_LAUNCH;
   }
 }

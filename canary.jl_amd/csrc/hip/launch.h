@@ -72,22 +72,22 @@ void launch_stage(int64_t nb, const KArgs& a) {
   constexpr int PF = (Phys::DIM == 3 && NQ == 7) ? 0 : 1;
   constexpr bool PM_LDS = true;
   constexpr int NT = FusedCfg<Phys, NQ, EPW, WIDE>::NT;
-  const int64_t chunk = (nb + 7) / 8;
-  stage_kernel<Phys, NQ, EPW, WIDE, PF, PM_LDS, MFMA><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, a.stream>>>(
+  const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
+  stage_kernel<Phys, NQ, EPW, WIDE, PF, PM_LDS, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.D, a.nreal, a.ntotal, a.vmapM, a.vmapP, a.bndy, a.rka, a.rkb,
-      a.dt, chunk, walk_back(a.Q, a.Qout), a.phys, a.advection);
+      a.dt, order, a.phys, a.advection);
 }
 
 template <class Phys, int NQ, int EPW, bool MFMA = false>
 void launch_stage_prep(int64_t nb, const KArgs& a) {
   constexpr int PF = (Phys::DIM == 3 && NQ == 7) ? 0 : 1;  // as launch_stage
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
-  const int64_t chunk = (nb + 7) / 8;
-  stage_prep_kernel<Phys, NQ, EPW, PF, MFMA><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, a.stream>>>(
+  const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
+  stage_prep_kernel<Phys, NQ, EPW, PF, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
-      (const double*)a.sgeo, a.pface, a.D, a.nreal, a.ntotal, a.rka, a.rkb, a.dt, chunk,
-      walk_back(a.Q, a.Qout), a.phys, a.advection);
+      (const double*)a.sgeo, a.pface, a.D, a.nreal, a.ntotal, a.rka, a.rkb, a.dt, order,
+      a.phys, a.advection);
 }
 
 // The prepared arrays hold no node heights: equation sets whose pressure
@@ -100,41 +100,42 @@ void launch_stage_prep_if(int64_t nb, const KArgs& a) {
 template <class Phys, int NQ, int EPW, bool MFMA>
 void launch_volume(int64_t nb, const KArgs& a) {
   constexpr int NT = VolumeCfg<Phys, NQ, EPW>::NT;
-  const int64_t chunk = (nb + 7) / 8;
-  volume_kernel<Phys, NQ, EPW, MFMA><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, a.stream>>>(
-      (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, a.D, a.nreal, chunk,
-      inplace_direction(), a.phys);
+  const BlockOrder order = block_order(nb, inplace_direction());
+  volume_kernel<Phys, NQ, EPW, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
+      (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, a.D, a.nreal, order,
+      a.phys);
 }
 
 template <class Phys, int NQ, int EPW>
 void launch_face(int64_t nb, const KArgs& a) {
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
-  const int64_t chunk = (nb + 7) / 8;
-  face_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, a.stream>>>(
+  const BlockOrder order = block_order(nb, inplace_direction());
+  face_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, (const double*)a.sgeo, a.nreal,
-      a.ntotal, a.vmapM, a.vmapP, a.bndy, chunk, inplace_direction(), a.phys);
+      a.ntotal, a.vmapM, a.vmapP, a.bndy, order, a.phys);
 }
 
 // Nonzero: the grid would not fit a launch.
 template <class Phys, int NQ>
 int launch_update(const KArgs& a) {
   const int64_t total = a.nreal * Shape<Phys, NQ>::Np;
-  const int64_t chunk = ((total + 255) / 256 + 7) / 8;
-  if (8 * chunk > 0x7fffffffLL) return 1;
-  update_kernel<Phys, NQ><<<dim3((unsigned)(8 * chunk)), dim3(256), 0, a.stream>>>(
+  const int64_t nb = (total + 255) / 256;
+  if (8 * ((nb + 7) / 8) > 0x7fffffffLL) return 1;
+  const BlockOrder order = block_order(nb, inplace_direction());
+  update_kernel<Phys, NQ><<<dim3((unsigned)(8 * order.chunk)), dim3(256), 0, a.stream>>>(
       (double*)a.rhs, (double*)a.Qout, (const double*)a.vgeo, a.nreal, a.rka, a.rkb, a.dt,
-      a.advection, chunk, inplace_direction());
+      a.advection, order);
   return 0;
 }
 
 template <class Phys, int NQ, int EPW>
 void launch_face_update(int64_t nb, const KArgs& a) {
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
-  const int64_t chunk = (nb + 7) / 8;
-  face_update_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, a.stream>>>(
+  const BlockOrder order = block_order(nb, inplace_direction());
+  face_update_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.nreal, a.ntotal, a.vmapM, a.vmapP, a.bndy, a.rka, a.rkb, a.dt,
-      chunk, inplace_direction(), a.phys, a.advection);
+      order, a.phys, a.advection);
 }
 
 // The operations a unit does not hold report CANARY_ERR_UNSUPPORTED.

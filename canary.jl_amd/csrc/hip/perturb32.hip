@@ -462,10 +462,10 @@ __global__ __launch_bounds__((Cfg32<DIM, NQ, single_epw<DIM, NQ>()>::NT)) void s
     float* __restrict__ rhs, const float* __restrict__ qin, float* __restrict__ qout,
     const float* __restrict__ bg, const float* __restrict__ vg, const float* __restrict__ sg,
     const int32_t* __restrict__ nbr, const double* __restrict__ D, int64_t nreal, float rka,
-    double bdt, int64_t chunk, int reverse, P32Params p) {
+    double bdt, BlockOrder order, P32Params p) {
   constexpr int EPW = single_epw<DIM, NQ>();
   __shared__ Lds32<DIM, NQ, EPW> L;
-  const int64_t e0 = stage_block(blockIdx.x, chunk, reverse) * EPW;
+  const int64_t e0 = stage_block(blockIdx.x, order) * EPW;
   if (e0 >= nreal) return;
   body<DIM, NQ, EPW>(L, rhs, qin, qout, bg, vg, sg, nbr, D, e0, nreal, (double)rka, bdt, p);
 }
@@ -476,10 +476,10 @@ __global__ __launch_bounds__((Cfg32<DIM, NQ, single_epw<DIM, NQ>()>::NT)) void s
     double* __restrict__ rhs, const float* __restrict__ qin, float* __restrict__ qout,
     const float* __restrict__ bg, const double* __restrict__ vg, const double* __restrict__ sg,
     const int32_t* __restrict__ nbr, const double* __restrict__ D, int64_t nreal, double rka,
-    double bdt, int64_t chunk, int reverse, P32Params p) {
+    double bdt, BlockOrder order, P32Params p) {
   constexpr int EPW = single_epw<DIM, NQ>();
   __shared__ Lds32<DIM, NQ, EPW> L;
-  const int64_t e0 = stage_block(blockIdx.x, chunk, reverse) * EPW;
+  const int64_t e0 = stage_block(blockIdx.x, order) * EPW;
   if (e0 >= nreal) return;
   body<DIM, NQ, EPW, double, double>(L, rhs, qin, qout, bg, vg, sg, nbr, D, e0, nreal, rka, bdt,
                                      p);
@@ -489,9 +489,9 @@ __global__ __launch_bounds__((Cfg32<DIM, NQ, single_epw<DIM, NQ>()>::NT)) void s
 template <int DIM, int NQ, int EPW>
 __global__ __launch_bounds__((Cfg32<DIM, NQ, EPW>::NT)) void batch32_kernel(
     const canary_p32_solve* __restrict__ solves, const canary_batch_item* __restrict__ items,
-    int64_t nitems, int64_t chunk, int parity, double rka, double rkb) {
+    int64_t nitems, BlockOrder order, int parity, double rka, double rkb) {
   __shared__ Lds32<DIM, NQ, EPW> L;
-  const int64_t w = stage_block(blockIdx.x, chunk, parity);  // direction alternates per stage
+  const int64_t w = stage_block(blockIdx.x, order);
   if (w >= nitems) return;
   const canary_batch_item it = items[w];
   const canary_p32_solve& sv = solves[it.solve];
@@ -542,12 +542,12 @@ int stage_mixed(void* rhs, const void* qin, void* qout, const void* bg, const vo
   constexpr int EPW = single_epw<DIM, NQ>();
   using C = Cfg32<DIM, NQ, EPW>;
   const int64_t nb = (nreal + EPW - 1) / EPW;
-  const int64_t chunk = (nb + 7) / 8;
+  // q ping-pong: the direction alternates
+  const BlockOrder order = block_order(nb, (uintptr_t)qin > (uintptr_t)qout ? 1 : 0);
   P32Params p{(float)ph->gamma, (float)(ph->c_p / ph->c_v), (float)ph->gravity};
-  stage_mixed_kernel<DIM, NQ><<<dim3((unsigned)(8 * chunk)), dim3(C::NT), 0, st>>>(
+  stage_mixed_kernel<DIM, NQ><<<dim3((unsigned)(8 * order.chunk)), dim3(C::NT), 0, st>>>(
       (double*)rhs, (const float*)qin, (float*)qout, (const float*)bg, (const double*)vg,
-      (const double*)sg, nbr, D, nreal, rka, rkb * dt, chunk,
-      (uintptr_t)qin > (uintptr_t)qout ? 1 : 0, p);
+      (const double*)sg, nbr, D, nreal, rka, rkb * dt, order, p);
   return launch_status();
 }
 
@@ -558,13 +558,12 @@ int stage(void* rhs, const void* qin, void* qout, const void* bg, const void* vg
   constexpr int EPW = single_epw<DIM, NQ>();
   using C = Cfg32<DIM, NQ, EPW>;
   const int64_t nb = (nreal + EPW - 1) / EPW;
-  const int64_t chunk = (nb + 7) / 8;
+  // q ping-pong: the direction alternates
+  const BlockOrder order = block_order(nb, (uintptr_t)qin > (uintptr_t)qout ? 1 : 0);
   P32Params p{(float)ph->gamma, (float)(ph->c_p / ph->c_v), (float)ph->gravity};
-  stage32_kernel<DIM, NQ><<<dim3((unsigned)(8 * chunk)), dim3(C::NT), 0, st>>>(
+  stage32_kernel<DIM, NQ><<<dim3((unsigned)(8 * order.chunk)), dim3(C::NT), 0, st>>>(
       (float*)rhs, (const float*)qin, (float*)qout, (const float*)bg, (const float*)vg,
-      (const float*)sg, nbr, D, nreal, (float)rka, rkb * dt, chunk,
-      (uintptr_t)qin > (uintptr_t)qout ? 1 : 0,  // q ping-pong: direction alternates
-      p);
+      (const float*)sg, nbr, D, nreal, (float)rka, rkb * dt, order, p);
   return launch_status();
 }
 
@@ -607,10 +606,10 @@ int batch_which(int* epw, int* threads, const canary_p32_solve* solves,
       *threads = NT;
       return 0;
     }
-    const int64_t chunk = (nitems + 7) / 8;
-    if (chunk > ((int64_t)1 << 27)) return CANARY_ERR_ARG;
-    batch32_kernel<DIM, NQ, E><<<dim3((unsigned)(8 * chunk)), dim3(NT), 0, st>>>(
-        solves, items, nitems, chunk, parity, rka, rkb);
+    if (nitems > ((int64_t)1 << 30)) return CANARY_ERR_ARG;
+    const BlockOrder order = block_order(nitems, parity);  // direction alternates per stage
+    batch32_kernel<DIM, NQ, E><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, st>>>(
+        solves, items, nitems, order, parity, rka, rkb);
     return launch_status();
   }
 }
