@@ -60,12 +60,68 @@ __device__ __forceinline__ void p32_error(unsigned long long code, long long fac
   }
 }
 
+// The stage was bound by VALU issue (0.9 of the cycles at 3D N=4 48^3: 1,098
+// instructions a wave, a third of them the library's log1p and expm1 and
+// IEEE divisions and roots).  The series and the refined hardware estimates
+// below take them to about 700 and leave it bound by memory: 2,265 -> 2,065 us
+// a step with the block order of dg_kernels.h, 1,974 with single_epw's blocks
+// (10.5 GB of least traffic, 5.3 TB/s).  Relative L2 error of one stage's
+// register against 64 bits, before -> after: ru 7.3e-8 the same, rv 7.1e-7 ->
+// 5.7e-7, rw 7.3e-7 -> 6.0e-7, rho and rho*theta the same.
+//
+// Pressure perturbation P' = P0 ((1 + x)^kappa - 1), x = rhotheta'/rhotheta0:
+// for |x| <= xmax the binomial series x (c[0] + x (c[1] + ...)),
+// c[i] = binom(kappa, i + 1), whose value comes without cancellation (x is a
+// factor); the first term left out, binom(kappa, 8) x^8, is below
+// 0.006 x^7 <= 3e-9 of the result for 1 <= kappa <= 2 and |x| <= 1/8 (a
+// twentieth of an FP32 rounding), so xmax is 1/8 for those kappa and
+// negative, i.e. no series, for any other.
+constexpr int kSeries = 7;
 struct P32Params {
-  float gamma, kappa, g;
+  float gamma, kappa, g, xmax;
+  float c[kSeries];
 };
 
-__device__ __forceinline__ P32Params params_of(const canary_phys& c) {
-  return P32Params{(float)c.gamma, (float)(c.c_p / c.c_v), (float)c.gravity};
+__host__ __device__ __forceinline__ P32Params params_of(const canary_phys& ph) {
+  P32Params p;
+  const double k = ph.c_p / ph.c_v;
+  p.gamma = (float)ph.gamma;
+  p.kappa = (float)k;
+  p.g = (float)ph.gravity;
+  p.xmax = k >= 1.0 && k <= 2.0 ? 0.125f : -1.f;
+  constexpr double inv[kSeries] = {1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 5, 1.0 / 6, 1.0 / 7, 1.0 / 8};
+  double b = k;
+#pragma unroll
+  for (int i = 0; i < kSeries; ++i) {
+    p.c[i] = (float)b;
+    b = b * (k - (i + 1)) * inv[i];
+  }
+  return p;
+}
+
+// The same values moved to scalar registers (every lane holds them).
+__device__ __forceinline__ P32Params scalar_params(P32Params p) {
+  static_assert(sizeof(P32Params) % 4 == 0, "words");
+  int w[sizeof(P32Params) / 4];
+  __builtin_memcpy(w, &p, sizeof(p));
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(P32Params) / 4; ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);
+  __builtin_memcpy(&p, w, sizeof(p));
+  return p;
+}
+
+// 1 / x and a / b by the hardware estimate (within an ulp) and one Newton
+// step in fused multiply-adds: within an ulp, a third of the instructions of
+// the IEEE division, whose scaling steps serve operands near the ends of the
+// exponent range (densities and rho*theta are not there).
+__device__ __forceinline__ float recip32(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return fmaf(fmaf(-x, r, 1.f), r, r);
+}
+// a / b, r the hardware estimate of 1 / b or recip32(b)
+__device__ __forceinline__ float div32(float a, float b, float r) {
+  const float q = a * r;
+  return fmaf(fmaf(-b, q, a), r, q);
 }
 
 template <int DIM>
@@ -91,8 +147,28 @@ __device__ __forceinline__ int fmask(int f, int fn) {
   }
 }
 
-__device__ __forceinline__ float pprime(float P0, float rt0, float rtp, float kappa) {
-  return P0 * expm1f(kappa * log1pf(rtp / rt0));
+// sqrt(x): the hardware root (within an ulp) and one Newton step where x is a
+// positive normal number (class mask 0x100); 0, infinity and NaN as the
+// hardware gives them.
+__device__ __forceinline__ float sqrt32(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float c = fmaf(fmaf(-s, s, x), 0.5f * __builtin_amdgcn_rsqf(x), s);
+  return __builtin_amdgcn_classf(x, 0x100) ? c : s;
+}
+
+// expm1(kappa log1p(x)) by the device library, out of line: the path outside
+// the series' range.
+__device__ __attribute__((noinline)) float expm1_klog1p(float x, float kappa) {
+  return expm1f(kappa * log1pf(x));
+}
+
+__device__ __forceinline__ float pprime(float P0, float rt0, float rtp, const P32Params& p) {
+  const float x = div32(rtp, rt0, __builtin_amdgcn_rcpf(rt0));
+  if (!(fabsf(x) <= p.xmax)) return P0 * expm1_klog1p(x, p.kappa);
+  float a = p.c[kSeries - 1];
+#pragma unroll
+  for (int i = kSeries - 2; i >= 0; --i) a = fmaf(a, x, p.c[i]);
+  return P0 * (x * a);
 }
 
 // ------------------------------------------------------------ prepare
@@ -207,17 +283,20 @@ struct Cfg32 {
   static constexpr int Np = ipow(NQ, DIM), Nfp = ipow(NQ, DIM - 1), NFN = 2 * DIM * Nfp;
   static constexpr int NT = round64(EPW * Np);
   static constexpr int FLUX = DIM * Np * NS;
-  static constexpr int POST = NFN * NS + Np * NS;
-  static constexpr int BUF = FLUX > POST ? FLUX : POST;
+  static constexpr int FACE = NFN * NS;
+  static constexpr int BUF = FLUX > FACE ? FLUX : FACE;
 };
 
 template <int DIM, int NQ, int EPW>
 struct Lds32 {
   using C = Cfg32<DIM, NQ, EPW>;
-  float D[NQ * NQ];
-  float Q[EPW][C::NS * C::Np];  // perturbation
-  float Bg[EPW][4 * C::Np];     // rho0, rhotheta0, P0, P'
-  float B[EPW][C::BUF];         // fluxes, then face terms + rhs
+  alignas(16) float B[EPW][C::BUF];  // fluxes, then face terms (then the FP64 register)
+  alignas(16) float D[NQ * NQ];
+  float Q[EPW][C::NS * C::Np];  // perturbation, then its result
+  union {
+    float Bg[EPW][4 * C::Np];      // rho0, rhotheta0, P0, P'
+    float R[EPW * C::NS * C::Np];  // the FP32 register's result
+  };
 };
 
 // Face record of the geometry word GT: (nx, ny, nz, sMJ) as floats.
@@ -308,7 +387,7 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
   if (t < NQ * NQ) L.D[t] = (float)dval;
   if (valid) {
     const float rho0 = b0, rt0 = b1, P0 = b2;
-    const float Pp = pprime(P0, rt0, q[E], p.kappa);
+    const float Pp = pprime(P0, rt0, q[E], p);
 #pragma unroll
     for (int s = 0; s < NS; ++s) L.Q[slot][s * Np + n] = q[s];
     L.Bg[slot][n] = rho0;
@@ -316,7 +395,7 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
     L.Bg[slot][2 * Np + n] = P0;
     L.Bg[slot][3 * Np + n] = Pp;
     const float rho = rho0 + q[RHO], rt = rt0 + q[E];
-    const float ri = 1.0f / rho;
+    const float ri = recip32(rho);
     // physical perturbation fluxes f[c][s] along coordinate c
     float f[DIM][NS];
 #pragma unroll
@@ -345,11 +424,7 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
     volume_sweeps<DIM, NQ, NS, float>(r, L.D, F0, F0 + NS * Np, F0 + (DIM > 2 ? 2 : 0) * NS * Np,
                                       n);
   }
-  lds_barrier();
-  if (valid) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) L.B[slot][NFN * NS + s * Np + n] = r[s];
-  }
+  lds_barrier();  // fluxes consumed: face terms take their place
   auto face = [&](int sl, int fi, const float* nn, float* qPl, int bc) {
     const int vid = fmask<DIM, NQ>(fi / Nfp, fi % Nfp);
     float qM[NS];
@@ -360,7 +435,7 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
     const float sMJ = nn[3];
     float PpP;
     if (bc == 0) {
-      PpP = pprime(P0, rt0, qPl[E], p.kappa);
+      PpP = pprime(P0, rt0, qPl[E], p);
     } else {
       float un = 0.f;
 #pragma unroll
@@ -379,9 +454,10 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
       UnM += nn[c] * qM[c];
       UnP += nn[c] * qPl[c];
     }
-    const float unM = UnM / rM, unP = UnP / rP;
-    const float lM = fabsf(unM) + sqrtf(p.gamma * (P0 + PpM) / rM);
-    const float lP = fabsf(unP) + sqrtf(p.gamma * (P0 + PpP) / rP);
+    const float rMi = recip32(rM), rPi = recip32(rP);
+    const float unM = UnM * rMi, unP = UnP * rPi;
+    const float lM = fabsf(unM) + sqrt32(div32(p.gamma * (P0 + PpM), rM, rMi));
+    const float lP = fabsf(unP) + sqrt32(div32(p.gamma * (P0 + PpP), rP, rPi));
     const float l = fmaxf(lM, lP);
     float nfM[NS], nfP[NS];
 #pragma unroll
@@ -419,42 +495,68 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
     face(sl, fi, nn, ql, bc);
   }
   lds_barrier();
+  // The node owner takes its own face terms, in ascending face order, and
+  // updates; its results go to LDS and from there out in storage order.
+  if (valid) {
+    const double MJI = FastOps::recip((double)MJg);  // the reference's MJI is 1 ./ MJ
+    const int ni = n % NQ, nj = (n / NQ) % NQ, nk = DIM == 3 ? n / (NQ * NQ) : 0;
+    const float* fc = L.B[slot];
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) {
-    for (int it = t; it < EPW * 2 * Nfp; it += NT) {
-      const int sl = it / (2 * Nfp), fi = 2 * d * Nfp + (it - sl * 2 * Nfp);
-      if (e0 + sl < nreal) {
-        const int v = fmask<DIM, NQ>(fi / Nfp, fi % Nfp);
-        float* rr = &L.B[sl][NFN * NS];
+    for (int d = 0; d < DIM; ++d) {
+      const int idx = d == 0 ? ni : (d == 1 ? nj : nk);
+      if (idx == 0 || idx == NQ - 1) {
+        const int fn = DIM == 2 ? (d == 0 ? nj : ni)
+                                : (d == 0 ? nj + NQ * nk : (d == 1 ? ni + NQ * nk : ni + NQ * nj));
+        const float* c = fc + ((2 * d + (idx != 0 ? 1 : 0)) * Nfp + fn) * NS;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) rr[s * Np + v] -= L.B[sl][fi * NS + s];
+        for (int s = 0; s < NS; ++s) r[s] -= c[s];
       }
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if constexpr (REG64) {
+        const double dq = (double)rreg[s] + (double)r[s];
+        L.Q[slot][s * Np + n] = (float)((double)q[s] + (bdt * dq) * MJI);
+        rreg[s] = rka * dq;
+      } else {
+        L.Q[slot][s * Np + n] = (float)((double)q[s] + (bdt * (double)r[s]) * MJI);
+        L.R[slot * NS * Np + s * Np + n] = (float)rka * r[s];
+      }
+    }
+  }
+  lds_barrier();
+  if constexpr (REG64) {  // the face terms are consumed: the FP64 register takes their place
+    if (valid) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        reinterpret_cast<double*>(&L.B[0][0])[slot * NS * Np + s * Np + n] = rreg[s];
     }
     lds_barrier();
   }
-  if (valid) {  // non-temporal stores: not read again in this stage
-    const double MJI = 1.0 / (double)MJg;  // the reference's MJI is 1 ./ MJ
-    float* qo = qout + (size_t)NS * Np * e;
-    RT* ro = rhs + (size_t)NS * Np * e;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const float rs = L.B[slot][NFN * NS + s * Np + n];
-      if constexpr (REG64) {
-        const double dq = (double)rreg[s] + (double)rs;
-        __builtin_nontemporal_store((float)((double)q[s] + (bdt * dq) * MJI), &qo[n + Np * s]);
-        __builtin_nontemporal_store(rka * dq, &ro[n + Np * s]);
-      } else {
-        __builtin_nontemporal_store((float)((double)q[s] + (bdt * (double)rs) * MJI),
-                                    &qo[n + Np * s]);
-        __builtin_nontemporal_store((float)rka * rs, &ro[n + Np * s]);
-      }
-    }
+  // Consecutive lanes write consecutive words (per-node stores write Np-word
+  // runs that start and end inside lines: 15% slower at 2D N=1, 4% at 2D N=4;
+  // 3D N=6 alone is 3% slower this way); non-temporal: nothing reads these
+  // lines again in this stage.
+  const int words = (nreal - e0 < EPW ? (int)(nreal - e0) : EPW) * NS * Np;
+  float* qo = qout + (size_t)NS * Np * (size_t)e0;
+  RT* ro = rhs + (size_t)NS * Np * (size_t)e0;
+  const RT* rs = REG64 ? reinterpret_cast<const RT*>(&L.B[0][0])
+                       : reinterpret_cast<const RT*>(&L.R[0]);
+  for (int i = t; i < words; i += NT) {
+    __builtin_nontemporal_store((&L.Q[0][0])[i], &qo[i]);
+    __builtin_nontemporal_store(rs[i], &ro[i]);
   }
 }
 
+// Elements per workgroup of the single-solve stage: as many as 256 lanes
+// hold.  The face items of a block then fill their last round of lanes
+// better (3D N=4: 300 items take 5 waves' rounds for two elements, 150 take 3
+// for one) and its writes have fewer ragged ends.  Against the fewest elements
+// that fill 90% of their lanes, us per step: 3D N=4 48^3 2065 -> 1974, 3D N=3
+// 50^3 1071 -> 1052, 2D N=4 500^2 661 -> 620, 2D N=2 800^2 743 -> 697.
 template <int DIM, int NQ>
 constexpr int single_epw() {
-  return default_epw<ipow(NQ, DIM)>();
+  return ipow(NQ, DIM) < 256 ? 256 / ipow(NQ, DIM) : 1;
 }
 
 template <int DIM, int NQ>
@@ -503,7 +605,7 @@ __global__ __launch_bounds__((Cfg32<DIM, NQ, EPW>::NT)) void batch32_kernel(
     if (threadIdx.x == 0) p32_error(1 /*CANARY_ERR_ARG*/, it.solve, it.e0 + 1, sv.nreal);
     return;
   }
-  const P32Params p = params_of(sv.phys);
+  const P32Params p = scalar_params(params_of(sv.phys));
   body<DIM, NQ, EPW>(L, (float*)sv.rhs, (const float*)sv.q[parity], (float*)sv.q[1 - parity],
                      (const float*)sv.bg32, (const float*)sv.vg, (const float*)sv.sg, sv.nbr,
                      sv.D, it.e0, sv.nreal, rka, rkb * sv.dt, p);
@@ -544,7 +646,7 @@ int stage_mixed(void* rhs, const void* qin, void* qout, const void* bg, const vo
   const int64_t nb = (nreal + EPW - 1) / EPW;
   // q ping-pong: the direction alternates
   const BlockOrder order = block_order(nb, (uintptr_t)qin > (uintptr_t)qout ? 1 : 0);
-  P32Params p{(float)ph->gamma, (float)(ph->c_p / ph->c_v), (float)ph->gravity};
+  const P32Params p = params_of(*ph);
   stage_mixed_kernel<DIM, NQ><<<dim3((unsigned)(8 * order.chunk)), dim3(C::NT), 0, st>>>(
       (double*)rhs, (const float*)qin, (float*)qout, (const float*)bg, (const double*)vg,
       (const double*)sg, nbr, D, nreal, rka, rkb * dt, order, p);
@@ -560,7 +662,7 @@ int stage(void* rhs, const void* qin, void* qout, const void* bg, const void* vg
   const int64_t nb = (nreal + EPW - 1) / EPW;
   // q ping-pong: the direction alternates
   const BlockOrder order = block_order(nb, (uintptr_t)qin > (uintptr_t)qout ? 1 : 0);
-  P32Params p{(float)ph->gamma, (float)(ph->c_p / ph->c_v), (float)ph->gravity};
+  const P32Params p = params_of(*ph);
   stage32_kernel<DIM, NQ><<<dim3((unsigned)(8 * order.chunk)), dim3(C::NT), 0, st>>>(
       (float*)rhs, (const float*)qin, (float*)qout, (const float*)bg, (const float*)vg,
       (const float*)sg, nbr, D, nreal, (float)rka, rkb * dt, order, p);
@@ -581,14 +683,14 @@ int reconstruct(int64_t nelem, const void* qp, const void* bg, void* Q, hipStrea
 constexpr int MAXT = 256;
 
 // candidate WHICH of elements per workgroup: 0 = most that fit MAXT
-// threads, 1 = about half of that, 2 = the single-solve choice; 0 = none
+// threads, 1 = about half of that, 2 = the first lane fill >= 90%; 0 = none
 template <int DIM, int NQ, int WHICH>
 constexpr int epw_candidate() {
   constexpr int Np = ipow(NQ, DIM);
   constexpr int emax = MAXT / Np;
   if (WHICH == 0) return emax > 0 ? emax : 1;  // more than MAXT nodes: one element alone
   if (WHICH == 1) return emax >= 2 ? (emax + 1) / 2 : 0;
-  if (WHICH == 2) return single_epw<DIM, NQ>() * Np <= MAXT ? single_epw<DIM, NQ>() : 0;
+  if (WHICH == 2) return default_epw<Np>() * Np <= MAXT ? default_epw<Np>() : 0;
   return 0;
 }
 
