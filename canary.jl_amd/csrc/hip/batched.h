@@ -70,16 +70,21 @@ __device__ __forceinline__ void solve_stage(char* lds, const canary_batch_solve&
                                             int parity, double rka, double rkb,
                                             const PhysParams& p) {
   using Real = typename Phys::Real;
+  Real* rhs = as_global((Real*)sv.rhs);
+  const Real* qin = as_global((const Real*)sv.Q[parity]);
+  Real* qout = as_global((Real*)sv.Q[1 - parity]);
+  const Real* vgeo = as_global((const Real*)sv.vgeo);
+  const Real* sgeo = as_global((const Real*)sv.sgeo);
+  const double* D = as_global(sv.D);
   if constexpr (PREP)
     stage_body<Phys, NQ, EPW, NT, PF, true, true, true, true>(
-        lds, (Real*)sv.rhs, (const Real*)sv.Q[parity], (Real*)sv.Q[1 - parity],
-        (const Real*)sv.vgeo, (const Real*)sv.sgeo, sv.D, e0, sv.nreal, sv.nelem_total, nullptr,
-        reinterpret_cast<const int64_t*>(sv.pface), nullptr, rka, rkb, sv.dt, p, sv.advection);
+        lds, rhs, qin, qout, vgeo, sgeo, D, e0, sv.nreal, sv.nelem_total, nullptr,
+        reinterpret_cast<const int64_t*>(as_global(sv.pface)), nullptr, rka, rkb, sv.dt, p,
+        sv.advection);
   else
     stage_body<Phys, NQ, EPW, NT, PF, true>(
-        lds, (Real*)sv.rhs, (const Real*)sv.Q[parity], (Real*)sv.Q[1 - parity],
-        (const Real*)sv.vgeo, (const Real*)sv.sgeo, sv.D, e0, sv.nreal, sv.nelem_total,
-        sv.vmapM, sv.vmapP, sv.elemtobndy, rka, rkb, sv.dt, p, sv.advection);
+        lds, rhs, qin, qout, vgeo, sgeo, D, e0, sv.nreal, sv.nelem_total, as_global(sv.vmapM),
+        as_global(sv.vmapP), as_global(sv.elemtobndy), rka, rkb, sv.dt, p, sv.advection);
 }
 
 // One workgroup per work-table entry, in the block order of stage_block (grid =

@@ -606,9 +606,10 @@ __global__ __launch_bounds__((Cfg32<DIM, NQ, EPW>::NT)) void batch32_kernel(
     return;
   }
   const P32Params p = scalar_params(params_of(sv.phys));
-  body<DIM, NQ, EPW>(L, (float*)sv.rhs, (const float*)sv.q[parity], (float*)sv.q[1 - parity],
-                     (const float*)sv.bg32, (const float*)sv.vg, (const float*)sv.sg, sv.nbr,
-                     sv.D, it.e0, sv.nreal, rka, rkb * sv.dt, p);
+  body<DIM, NQ, EPW>(L, as_global((float*)sv.rhs), as_global((const float*)sv.q[parity]),
+                     as_global((float*)sv.q[1 - parity]), as_global((const float*)sv.bg32),
+                     as_global((const float*)sv.vg), as_global((const float*)sv.sg),
+                     as_global(sv.nbr), as_global(sv.D), it.e0, sv.nreal, rka, rkb * sv.dt, p);
 }
 
 int launch_status() { return hipGetLastError() == hipSuccess ? 0 : CANARY_ERR_LAUNCH; }
