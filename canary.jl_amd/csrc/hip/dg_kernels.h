@@ -153,6 +153,13 @@ __device__ __forceinline__ T* as_global(T* p) {
   return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
 }
 
+// a + x * y: in FP64 as the unit contracts it (the exact-order units do not),
+// in FP32 fused.
+__device__ __forceinline__ double mul_add(double x, double y, double a) { return a + x * y; }
+__device__ __forceinline__ float mul_add(float x, float y, float a) { return fmaf(x, y, a); }
+__device__ __forceinline__ double one_over(double x) { return 1.0 / x; }
+__device__ __forceinline__ float one_over(float x) { return recip32(x); }
+
 // ------------------------------------------------------------------ sweeps
 // r[s] += sum_m D[m, i] F[m, j, k, s] (xi), then eta, then zeta, with the
 // reference CPU order.  sF[d] points at the flux of direction d,
@@ -171,12 +178,12 @@ __device__ __forceinline__ void volume_sweeps(Real* r, const Real* sD, const Rea
   for (int s = 0; s < NSR; ++s) {
     Real a = r[s];
 #pragma unroll
-    for (int m = 0; m < NQ; ++m) a = a + sD[m + NQ * i] * sF0[s * Np + base_xi + m];
+    for (int m = 0; m < NQ; ++m) a = mul_add(sD[m + NQ * i], sF0[s * Np + base_xi + m], a);
 #pragma unroll
-    for (int m = 0; m < NQ; ++m) a = a + sD[m + NQ * j] * sF1[s * Np + base_eta + m * NQ];
+    for (int m = 0; m < NQ; ++m) a = mul_add(sD[m + NQ * j], sF1[s * Np + base_eta + m * NQ], a);
     if (DIM == 3) {
 #pragma unroll
-      for (int m = 0; m < NQ; ++m) a = a + sD[m + NQ * k] * sF2[s * Np + base_zeta + m * NQ * NQ];
+      for (int m = 0; m < NQ; ++m) a = mul_add(sD[m + NQ * k], sF2[s * Np + base_zeta + m * NQ * NQ], a);
     }
     r[s] = a;
   }
@@ -194,7 +201,7 @@ __device__ __forceinline__ void volume_sweep_dir(Real* r, const Real* sD, const 
   for (int s = 0; s < NSR; ++s) {
     Real a = r[s];
 #pragma unroll
-    for (int m = 0; m < NQ; ++m) a = a + sD[m + NQ * idx] * sF[s * Np + base + m * STRIDE];
+    for (int m = 0; m < NQ; ++m) a = mul_add(sD[m + NQ * idx], sF[s * Np + base + m * STRIDE], a);
     r[s] = a;
   }
 }
@@ -898,7 +905,8 @@ __device__ __forceinline__ void stage_body(
   //    Hu = (h + b) u after it (shallow_water.jl:274-297).
   if (UPDATE && valid) {
     // prepared arrays hold no MJI: the reference's is 1 ./ MJ (IEEE division)
-    if constexpr (PREP) MJI = Real(1) / MJ;
+    // (FP32: refined estimate)
+    if constexpr (PREP) MJI = one_over(MJ);
     const Real bdt = (Real)(rkb * dt);
     const Real ka = (Real)rka;
     Real* qn = sQ + slot * NS * Np + n;
@@ -916,7 +924,7 @@ __device__ __forceinline__ void stage_body(
     for (int s = 0; s < NSR; ++s) {
       Real& qq = qn[s * Np];
       const Real rs = rv[s];
-      qq = qq + bdt * rs * MJI;
+      qq = mul_add(bdt * rs, MJI, qq);
       sB[slot * BUF + NFN * NSR + s * Np + n] = rs * ka;
     }
     if (Phys::HAS_ADVECTION && advection) {

@@ -110,20 +110,6 @@ __device__ __forceinline__ P32Params scalar_params(P32Params p) {
   return p;
 }
 
-// 1 / x and a / b by the hardware estimate (within an ulp) and one Newton
-// step in fused multiply-adds: within an ulp, a third of the instructions of
-// the IEEE division, whose scaling steps serve operands near the ends of the
-// exponent range (densities and rho*theta are not there).
-__device__ __forceinline__ float recip32(float x) {
-  const float r = __builtin_amdgcn_rcpf(x);
-  return fmaf(fmaf(-x, r, 1.f), r, r);
-}
-// a / b, r the hardware estimate of 1 / b or recip32(b)
-__device__ __forceinline__ float div32(float a, float b, float r) {
-  const float q = a * r;
-  return fmaf(fmaf(-b, q, a), r, q);
-}
-
 template <int DIM>
 struct Dims {
   static constexpr int NS = DIM + 2;            // U, V, (W), rho, rhotheta
@@ -145,15 +131,6 @@ __device__ __forceinline__ int fmask(int f, int fn) {
     case 1: return a + NQ * ((f & 1) * N) + NQ * NQ * b;
     default: return a + NQ * b + NQ * NQ * ((f & 1) * N);
   }
-}
-
-// sqrt(x): the hardware root (within an ulp) and one Newton step where x is a
-// positive normal number (class mask 0x100); 0, infinity and NaN as the
-// hardware gives them.
-__device__ __forceinline__ float sqrt32(float x) {
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float c = fmaf(fmaf(-s, s, x), 0.5f * __builtin_amdgcn_rsqf(x), s);
-  return __builtin_amdgcn_classf(x, 0x100) ? c : s;
 }
 
 // expm1(kappa log1p(x)) by the device library, out of line: the path outside
