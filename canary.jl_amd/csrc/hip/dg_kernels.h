@@ -20,10 +20,9 @@
 // the correctly rounded pow of crpow.h (the oracle's pow is correctly
 // rounded too) the exact-order kernels give the oracle's bits.
 //
-// Face contributions are scattered into a staged copy of the element's rhs
-// in LDS in `DIM` rounds, faces (2d, 2d+1) per round: the two faces of one
-// direction share no node, so the owner computes without atomics, and edge
-// and corner nodes receive their face terms in ascending face order.
+// Face terms are left in LDS and taken by each node's own thread, which knows
+// its one to DIM face items from its indices: no atomics, and edge and corner
+// nodes receive their face terms in ascending face order.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -251,33 +250,41 @@ __device__ __forceinline__ int canon_vid(int f, int fn) {
   }
 }
 
-// face_meta in two halves: face_load issues the loads (no use of their
-// values, so a kernel can issue more loads behind them), face_resolve checks
-// the maps and bc and splits the node ids.
+// face_meta in parts: face_load_maps and face_load_geo issue the loads (no
+// use of their values, so a kernel can issue more loads behind them),
+// face_resolve checks the maps and bc and splits the node ids.
 //
 // A null vmapM stands for the canonical face mask (the only vmapM that
 // src/mesh.jl builds): the M-side id is computed, and the map load re-reads
 // the vmapP entry instead (a cache hit, no HBM bytes), so both forms run one
 // instruction sequence in one kernel.
 template <class Phys, int NQ>
-__device__ __forceinline__ void face_load(FaceItem<Phys>& it,
-                                          const typename Phys::Real* __restrict__ sgeo,
-                                          const int64_t* __restrict__ vmapM,
-                                          const int64_t* __restrict__ vmapP,
-                                          const int64_t* __restrict__ bndy, int64_t e, int fi) {
+__device__ __forceinline__ void face_load_maps(FaceItem<Phys>& it,
+                                               const int64_t* __restrict__ vmapM,
+                                               const int64_t* __restrict__ vmapP,
+                                               const int64_t* __restrict__ bndy, int64_t e,
+                                               int fi) {
   using S = Shape<Phys, NQ>;
-  constexpr int DIM = Phys::DIM, NSG = Phys::NSGEO;
+  constexpr int DIM = Phys::DIM;
   const int f = fi / S::Nfp;
   const size_t fo = (size_t)fi + (size_t)S::NFN * (size_t)e;
-  const typename Phys::Real* sg = sgeo + (size_t)NSG * fo;
-#pragma unroll
-  for (int c = 0; c < DIM; ++c) it.nrm[c] = sg[c];
-  it.sMJ = sg[DIM];
   const bool canon = vmapM == nullptr;
   const int64_t rawM = (canon ? vmapP : vmapM)[fo];
   it.idP = vmapP[fo];
   it.idM = canon ? (int64_t)S::Np * e + canon_vid<DIM, NQ>(f, fi - f * S::Nfp) + 1 : rawM;
   it.bcode = bndy[f + S::NFACE * e];
+}
+
+// normal and sMJ of face item fi of element e, NSG words a record
+template <class Phys, int NQ, int NSG>
+__device__ __forceinline__ void face_load_geo(FaceItem<Phys>& it,
+                                              const typename Phys::Real* __restrict__ sgeo,
+                                              int64_t e, int fi) {
+  constexpr int DIM = Phys::DIM, NFN = Shape<Phys, NQ>::NFN;
+  const typename Phys::Real* sg = sgeo + (size_t)NSG * ((size_t)fi + (size_t)NFN * (size_t)e);
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) it.nrm[c] = sg[c];
+  it.sMJ = sg[DIM];
 }
 
 // The maps are split and selected without branching on them (a load whose
@@ -322,7 +329,8 @@ __device__ __forceinline__ void face_meta(FaceItem<Phys>& it,
                                           const int64_t* __restrict__ vmapP,
                                           const int64_t* __restrict__ bndy, int64_t e, int fi,
                                           int64_t ntotal) {
-  face_load<Phys, NQ>(it, sgeo, vmapM, vmapP, bndy, e, fi);
+  face_load_maps<Phys, NQ>(it, vmapM, vmapP, bndy, e, fi);
+  face_load_geo<Phys, NQ, Phys::NSGEO>(it, sgeo, e, fi);
   face_resolve<Phys, NQ>(it, e, fi, ntotal);
 }
 
@@ -343,22 +351,14 @@ struct Prepared {
   static constexpr int NSG = DIM + 1;       // psgeo fields
 };
 
-// face_load over the prepared arrays: the face code goes to idP and is
+// face_load_maps over the prepared arrays: the face code goes to idP and is
 // turned into node ids by face_decode_resolve once it has arrived.
 template <class Phys, int NQ>
-__device__ __forceinline__ void face_load_prep(FaceItem<Phys>& it,
-                                               const typename Phys::Real* __restrict__ psgeo,
+__device__ __forceinline__ void face_load_code(FaceItem<Phys>& it,
                                                const int32_t* __restrict__ pface, int64_t e,
                                                int fi) {
   using S = Shape<Phys, NQ>;
-  constexpr int DIM = Phys::DIM, NSG = Prepared<Phys>::NSG;
-  const int f = fi / S::Nfp;
-  const size_t fo = (size_t)fi + (size_t)S::NFN * (size_t)e;
-  const typename Phys::Real* sg = psgeo + (size_t)NSG * fo;
-#pragma unroll
-  for (int c = 0; c < DIM; ++c) it.nrm[c] = sg[c];
-  it.sMJ = sg[DIM];
-  it.idP = pface[f + S::NFACE * e];
+  it.idP = pface[fi / S::Nfp + S::NFACE * e];
 }
 
 // face_decode + face_resolve over the prepared arrays, without building the
@@ -500,6 +500,19 @@ __device__ __forceinline__ void face_terms_at_node(Real* r, const Real* sC, cons
   }
 }
 
+// The same when vmapM is not the canonical face mask: the node owner looks
+// through every item's node in ascending order.
+template <int NFN, int NSR, class Real, class VidT>
+__device__ __forceinline__ void face_terms_by_search(Real* r, const Real* sC, const VidT* sV,
+                                                     int n) {
+#pragma unroll 1
+  for (int fi = 0; fi < NFN; ++fi)
+    if (sV[fi] == (VidT)n) {
+#pragma unroll
+      for (int s = 0; s < NSR; ++s) r[s] = r[s] - sC[fi * NSR + s];
+    }
+}
+
 // ================================================================ kernels
 template <class Phys, int NQ, int EPW>
 struct VolumeCfg {
@@ -625,17 +638,16 @@ __global__ __launch_bounds__(256) void update_kernel(double* __restrict__ rhs,
 // Qout; rhs in place.
 //
 // Schedule (per workgroup):
-//   1. each thread issues the loads of its first face item (maps, normals,
-//      bc), of D and of its volume node's Q, metric terms and rhs, before
-//      it uses any of them;
-//   2. the P-side gather of the face item is issued as soon as its map has
-//      arrived; volume fluxes -> LDS;
-//   3. the xi/eta/zeta sweeps run from LDS while the gathers are in flight
-//      (barriers fence LDS only, so loads stay outstanding across them);
-//   4. face fluxes -> LDS, taken into the staged rhs by each node's thread
-//      in ascending face order (or scattered in DIM rounds when vmapM is not
-//      the canonical face mask);
-//   5. update: Qout = Q + ((rkb*dt)*rhs)*MJI, rhs *= rka, in LDS;
+//   1. each thread issues the loads of its first face item (maps, bc; unless
+//      gather_late its normal and sMJ), of D and of its volume node's Q,
+//      metric terms and rhs, before it uses any of them;
+//   2. volume fluxes in registers; the P-side gather of the face item before
+//      them, as soon as its map has arrived, or (gather_late) after them;
+//   3. the xi/eta/zeta sweeps run through one flux buffer in LDS while the
+//      gathers are in flight (barriers fence LDS only, so loads stay
+//      outstanding across them); rhs accumulates in registers;
+//   4. face fluxes -> LDS, taken by each node's thread in ascending face order;
+//   5. update: Qout = Q + ((rkb*dt)*rhs)*MJI, rhs *= rka, to LDS;
 //   6. the block's Qout and rhs written out in storage order.
 template <class Phys, int NQ, int EPW, bool WIDE>
 struct FusedCfg {
@@ -648,8 +660,8 @@ struct FusedCfg {
   static constexpr int NFACEIT = round64(EPW * S::NFN);
   static constexpr int NT = WIDE && NFACEIT > NVOL ? NFACEIT : NVOL;
   static constexpr int FLUX = S::Np;                       // per state, one direction
-  static constexpr int POST = S::NFN + S::Np;               // sC + sR per state
-  static constexpr int BUF = (FLUX > POST ? FLUX : POST) * Phys::NSR;
+  static constexpr int FACE = S::NFN + S::Np;               // face terms + rhs per state
+  static constexpr int BUF = (FLUX > FACE ? FLUX : FACE) * Phys::NSR;
   // LDS carve-up (bytes, each piece 16-byte aligned)
   static constexpr int a16(int b) { return (b + 15) / 16 * 16; }
   static constexpr int OFF_D = 0;
@@ -660,6 +672,33 @@ struct FusedCfg {
   static constexpr int OFF_F = OFF_V + a16(sizeof(VidT) * EPW * S::NFN);  // one flag word
   static constexpr int LDS = OFF_F + 16;
 };
+
+// When a stage issues its face items' geometry and P-side gathers: before the
+// volume fluxes, so that they have the longest time to arrive, or (LATE) after
+// them, in flight over the sweeps, so that their registers are not live with
+// the metric terms.  LATE pays where registers limit the waves that fit: the
+// exact-order 3D kernels (32^3 N=4, reference arrays: 1,422 -> 1,377 us a step;
+// N=7: 1,342 -> 1,235) and the contracted ones from N = 6 on; the contracted
+// ones below are faster early (N=5: 1,042 against 1,058), as is 2D (10 x 10
+// meshes wait for latency alone: 240 against 269 us for 50 stages).
+//
+// 3D N = 6 has 343 nodes in six waves: at 96 VGPRs five waves fit a SIMD and
+// three workgroups a CU, above that two.  It is built for that (stage_waves),
+// with the maps read after the fluxes too (MAPS_LATE) and rhs left in LDS
+// over the face phase; without these it spills.  23^3 stage 348 -> 304 us,
+// prepared loop exact 1,619 -> 1,416, contracted 1,302 -> 1,137.
+template <class Phys, int NQ>
+constexpr bool gather_late() {
+  if constexpr (Phys::DIM == 3)
+    return Phys::EXACT || NQ >= 7;
+  else
+    return false;
+}
+
+template <class Phys, int NQ>
+constexpr int stage_waves() {  // waves a SIMD must hold
+  return Phys::DIM == 3 && NQ == 7 ? 5 : 1;
+}
 
 // One fused stage of the EPW-element block starting at e0, computed by NT
 // threads (NT >= the volume nodes of the block).  `lds` holds
@@ -693,6 +732,11 @@ __device__ __forceinline__ void stage_body(
   // prepared arrays: psgeo in `sgeo`, the face codes in `vmapP`'s place
   const int32_t* __restrict__ pface = reinterpret_cast<const int32_t*>(vmapP);
   constexpr int KP = PF < KF ? PF : KF;
+  constexpr bool LATE = VOLUME && gather_late<Phys, NQ>();
+  constexpr bool N6 = stage_waves<Phys, NQ>() > 1;
+  constexpr bool MAPS_LATE = LATE && !PREP && N6;
+  constexpr bool STAGE_R = !VOLUME || N6;  // rhs waits in LDS for the face terms
+  constexpr int NSG = PREP ? Prepared<Phys>::NSG : Phys::NSGEO;
   constexpr bool SP = Phys::HAS_P && PM_LDS;
   constexpr int BUF = C::BUF;
   using VidT = typename C::VidT;
@@ -708,74 +752,76 @@ __device__ __forceinline__ void stage_body(
   int* sFlag = reinterpret_cast<int*>(lds + C::OFF_F);  // a non-canonical M-side node seen
 
   const int t = threadIdx.x;
-  const int slot = t / Np, n = t - slot * Np;
-  const int64_t e = e0 + slot;
-  const bool valid = slot < EPW && e < nreal;
+  const int slot = EPW == 1 ? 0 : t / Np, n = t - slot * Np;
+  const bool valid = EPW == 1 ? t < Np : slot < EPW && e0 + slot < nreal;
 
-  // 1. issue every load of the block before any of them is used: the face
-  //    items' normals, maps and bc (t, t + NT, ...), D, the node's Q, metric
-  //    terms and rhs -- one memory round trip instead of one per kind.  The
-  //    loads are unconditional (lanes without work read in-bounds element
-  //    e0, node 0, and ignore it): a load under a branch makes every later
-  //    wait count for the path without it, i.e. wait for everything.
+  // 1. issue the loads of the block before any of them is used: the face
+  //    items' maps and bc (t, t + NT, ...), D, the node's Q, metric terms and
+  //    rhs -- one memory round trip instead of one per kind.  The loads are
+  //    unconditional (lanes without work read in-bounds element e0, node 0,
+  //    and ignore it): a load under a branch makes every later wait count
+  //    for the path without it, i.e. wait for everything.
   FaceItem<Phys> fit[KP > 0 ? KP : 1];  // KP = 0: every face item after the volume work
   bool fval[KP > 0 ? KP : 1];
+  int fsl[KP > 0 ? KP : 1], ffi[KP > 0 ? KP : 1];
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
     const int item = t + k * NT;
-    const int sl = item / NFN;
-    fval[k] = item < EPW * NFN && e0 + sl < nreal;
+    fsl[k] = EPW == 1 ? 0 : item / NFN;
+    fval[k] = item < EPW * NFN && (EPW == 1 || e0 + fsl[k] < nreal);
+    fsl[k] = fval[k] ? fsl[k] : 0;
+    ffi[k] = fval[k] ? item - fsl[k] * NFN : 0;
     if constexpr (PREP)
-      face_load_prep<Phys, NQ>(fit[k], sgeo, pface, fval[k] ? e0 + sl : e0,
-                               fval[k] ? item - sl * NFN : 0);
-    else
-      face_load<Phys, NQ>(fit[k], sgeo, vmapM, vmapP, bndy, fval[k] ? e0 + sl : e0,
-                          fval[k] ? item - sl * NFN : 0);
+      face_load_code<Phys, NQ>(fit[k], pface, e0 + fsl[k], ffi[k]);
+    else if constexpr (!MAPS_LATE)
+      face_load_maps<Phys, NQ>(fit[k], vmapM, vmapP, bndy, e0 + fsl[k], ffi[k]);
+    if constexpr (!LATE) face_load_geo<Phys, NQ, NSG>(fit[k], sgeo, e0 + fsl[k], ffi[k]);
   }
   double dval = 0.0;
   if constexpr (VOLUME) dval = D[t < NQ * NQ ? t : 0];
   // keep the map loads ahead of the node loads: waiting for the maps then
   // leaves the node loads in flight (the wait counter is in issue order)
   __builtin_amdgcn_sched_barrier(0);
-  const int64_t el = valid ? e : e0;
-  const int nl = valid ? n : 0;
+  const int sl0 = valid ? slot : 0, nl = valid ? n : 0;
+  const int64_t el = e0 + sl0;
   Real q[NS], met[DIM * DIM], r[NSR];
-  const Real* qe = Qin + (size_t)NS * Np * (size_t)el;
+  const Real* qe = Qin + (size_t)NS * Np * (size_t)e0 + (sl0 * NS * Np + nl);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) q[s] = qe[nl + Np * s];
-  const Real* vg = (VOLUME || UPDATE) ? vgeo + (size_t)NV * Np * (size_t)el : nullptr;
+  for (int s = 0; s < NS; ++s) q[s] = qe[Np * s];
+  const Real* vg = (VOLUME || UPDATE)
+                       ? vgeo + (size_t)NV * Np * (size_t)e0 + (sl0 * NV * Np + nl)
+                       : nullptr;
   // the node's height, for a pressure that needs it (loaded with the rest)
   const Real ynode = NeedsY<Phys>::value ? node_y<Phys, NQ>(vgeo, el, nl) : Real(0);
   Real MJ = 0;
   if constexpr (VOLUME) {
 #pragma unroll
-    for (int c = 0; c < DIM * DIM; ++c) met[c] = vg[nl + Np * c];
-    MJ = vg[nl + Np * Phys::iMJ];
+    for (int c = 0; c < DIM * DIM; ++c) met[c] = vg[Np * c];
+    MJ = vg[Np * Phys::iMJ];
   }
-  Real MJI = 0;
-  if constexpr (UPDATE && !PREP) MJI = vg[nl + Np * Phys::iMJI];
-  const Real* re = rhs + (size_t)NS * Np * (size_t)el;
+  const Real* re = rhs + (size_t)NS * Np * (size_t)e0 + (sl0 * NS * Np + nl);
 #pragma unroll
-  for (int s = 0; s < NSR; ++s) r[s] = re[nl + Np * s];
-  // 2. maps checked as soon as they arrive and the P-side gathers issued
-  //    (unconditionally, as above: lanes without an item check the item
-  //    they loaded, e0's first face node, which some lane owns anyway);
-  //    the gathers stay in flight over the volume work and the sweeps
+  for (int s = 0; s < NSR; ++s) r[s] = re[Np * s];
+  // maps checked as soon as they arrive and the P-side gathers issued
+  // (unconditionally, as above: lanes without an item check the item
+  // they loaded, e0's first face node, which some lane owns anyway)
+  auto gather = [&]() {
 #pragma unroll
-  for (int k = 0; k < KP; ++k) {
-    const int item = t + k * NT;
-    const int sl = item / NFN;
-    if constexpr (PREP)
-      face_decode_resolve<Phys, NQ>(fit[k], fval[k] ? e0 + sl : e0,
-                                    fval[k] ? item - sl * NFN : 0, ntotal);
-    else
-      face_resolve<Phys, NQ>(fit[k], fval[k] ? e0 + sl : e0, fval[k] ? item - sl * NFN : 0,
-                             ntotal);
-    face_gather_any<Phys, NQ>(fit[k], Qin, vgeo, fval[k], e0);
-  }
+    for (int k = 0; k < KP; ++k) {
+      if constexpr (LATE && !MAPS_LATE)
+        face_load_geo<Phys, NQ, NSG>(fit[k], sgeo, e0 + fsl[k], ffi[k]);
+      if constexpr (PREP)
+        face_decode_resolve<Phys, NQ>(fit[k], e0 + fsl[k], ffi[k], ntotal);
+      else
+        face_resolve<Phys, NQ>(fit[k], e0 + fsl[k], ffi[k], ntotal);
+      face_gather_any<Phys, NQ>(fit[k], Qin, vgeo, fval[k], e0);
+    }
+  };
+  if constexpr (!LATE) gather();
 
   if (VOLUME && t < NQ * NQ) sD[t] = (Real)dval;
   if (!PREP && t == 0) *sFlag = 0;  // read after the face terms, barriers later
+  // 2. volume fluxes
   Real Fv[DIM][NSR];
   if (valid) {
 #pragma unroll
@@ -787,6 +833,21 @@ __device__ __forceinline__ void stage_body(
       Phys::source(q, MJ, p, r);
     }
   }
+  if constexpr (LATE) {
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MAPS_LATE) {
+#pragma unroll
+      for (int k = 0; k < KP; ++k) {
+        face_load_maps<Phys, NQ>(fit[k], vmapM, vmapP, bndy, e0 + fsl[k], ffi[k]);
+        face_load_geo<Phys, NQ, NSG>(fit[k], sgeo, e0 + fsl[k], ffi[k]);
+      }
+    } else {
+      gather();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  Real MJI = 0;
+  if constexpr (UPDATE && !PREP && !MAPS_LATE) MJI = vg[Np * Phys::iMJI];
   // 3. sweeps, one direction at a time through one flux buffer
 #pragma unroll
   for (int d = 0; d < (VOLUME ? DIM : 0); ++d) {
@@ -814,11 +875,20 @@ __device__ __forceinline__ void stage_body(
       if (d == 1) volume_sweep_dir<DIM, NQ, NSR, Real, (DIM > 1 ? 1 : 0)>(r, sD, b, n);
       if (d == 2) volume_sweep_dir<DIM, NQ, NSR, Real, (DIM > 2 ? 2 : 0)>(r, sD, b, n);
     }
+    if constexpr (MAPS_LATE) {
+      if (d == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        gather();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
   }
-  lds_barrier();  // fluxes consumed; sB is reused below
-  if (valid) {
+  lds_barrier();  // fluxes consumed (and Q, P staged): face terms take their place
+  if constexpr (STAGE_R) {
+    if (valid) {
 #pragma unroll
-    for (int s = 0; s < NSR; ++s) sB[slot * BUF + NFN * NSR + s * Np + n] = r[s];
+      for (int s = 0; s < NSR; ++s) sB[slot * BUF + NFN * NSR + s * Np + n] = r[s];
+    }
   }
   // 4. face fluxes: M side from LDS, P side gathered
   bool noncanon = false;  // an item whose M-side node is not the canonical one
@@ -832,8 +902,7 @@ __device__ __forceinline__ void stage_body(
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
     if (!fval[k]) continue;
-    const int item = t + k * NT;
-    const int sl = item / NFN, fi = item - sl * NFN;
+    const int sl = fsl[k], fi = ffi[k];
     auto qm_at = [&](int s, int v) { return sQ[sl * NS * Np + s * Np + v]; };
     auto pm_at = [&](int v, const Real* qm) { return pm_of(sl, v, qm); };
     Real c[NSR];
@@ -844,15 +913,16 @@ __device__ __forceinline__ void stage_body(
     for (int s = 0; s < NSR; ++s) sB[sl * BUF + fi * NSR + s] = c[s];
   }
   for (int item = t + KP * NT; item < EPW * NFN; item += NT) {
-    const int sl = item / NFN, fi = item - sl * NFN;
-    if (e0 + sl >= nreal) continue;
+    const int sl = EPW == 1 ? 0 : item / NFN, fi = item - sl * NFN;
+    if (EPW > 1 && e0 + sl >= nreal) continue;
     auto qm_at = [&](int s, int v) { return sQ[sl * NS * Np + s * Np + v]; };
     auto pm_at = [&](int v, const Real* qm) { return pm_of(sl, v, qm); };
     Real c[NSR];
     int vid;
     if constexpr (PREP) {
       FaceItem<Phys> it;
-      face_load_prep<Phys, NQ>(it, sgeo, pface, e0 + sl, fi);
+      face_load_code<Phys, NQ>(it, pface, e0 + sl, fi);
+      face_load_geo<Phys, NQ, NSG>(it, sgeo, e0 + sl, fi);
       face_decode_resolve<Phys, NQ>(it, e0 + sl, fi, ntotal);
       face_gather<Phys, NQ>(it, Qin, vgeo);
       vid = face_finish<Phys>(it, p, qm_at, pm_at, c);
@@ -865,73 +935,54 @@ __device__ __forceinline__ void stage_body(
 #pragma unroll
     for (int s = 0; s < NSR; ++s) sB[sl * BUF + fi * NSR + s] = c[s];
   }
-  // The face terms reach rhs (staged in LDS) in ascending face order: with
-  // the canonical face mask (always over the prepared arrays; over the
-  // reference arrays when every item of the workgroup maps to its canonical
-  // node) the node owner gathers its own (face_terms_at_node, no barrier);
-  // else the face pairs are scattered round by round.  Same operations in
-  // the same order either way.
   if (!PREP && noncanon) *sFlag = 1;
   lds_barrier();
-  const bool scatter = !PREP && *sFlag != 0;
-  if (scatter) {
+  // 5. each node's thread takes its own face terms in ascending face order
+  //    (with the canonical face mask, always so over the prepared arrays, it
+  //    finds them from its indices; over the reference arrays, in a workgroup
+  //    with any other vmapM, it looks through the items' nodes), then updates.
+  //    Shallow water with `advection` keeps the velocity: u = Hu / (h + b)
+  //    before the update, Hu = (h + b) u after it (shallow_water.jl:274-297).
+  if (valid) {
+    if constexpr (STAGE_R) {
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      for (int it = t; it < EPW * 2 * Nfp; it += NT) {
-        const int sl = it / (2 * Nfp), fi = 2 * d * Nfp + (it - sl * 2 * Nfp);
-        const VidT v = sV[sl * NFN + fi];
-        if (e0 + sl < nreal && v != NOVID) {
-          Real* rr = sB + sl * BUF + NFN * NSR;
-#pragma unroll
-          for (int s = 0; s < NSR; ++s)
-            rr[s * Np + v] = rr[s * Np + v] - sB[sl * BUF + fi * NSR + s];
-        }
+      for (int s = 0; s < NSR; ++s) r[s] = sB[slot * BUF + NFN * NSR + s * Np + n];
+    }
+    if (!PREP && *sFlag != 0)
+      face_terms_by_search<NFN, NSR>(r, sB + slot * BUF, sV + slot * NFN, n);
+    else
+      face_terms_at_node<DIM, NQ, NSR>(r, sB + slot * BUF, sV + slot * NFN, n, NOVID);
+    if constexpr (UPDATE) {
+      // prepared arrays hold no MJI: the reference's is 1 ./ MJ (IEEE division;
+      // FP32: refined estimate)
+      if constexpr (PREP) MJI = one_over(MJ);
+      if constexpr (MAPS_LATE) MJI = vg[Np * Phys::iMJI];
+      const Real bdt = (Real)(rkb * dt);
+      const Real ka = (Real)rka;
+      Real* qn = sQ + slot * NS * Np + n;
+      Real uu = 0, vv = 0;
+      if (Phys::HAS_ADVECTION && advection) {
+        const Real Ht = qn[Np * 2] + qn[Np * 3];
+        uu = qn[0] / Ht;
+        vv = qn[Np] / Ht;
       }
-      lds_barrier();
+#pragma unroll
+      for (int s = 0; s < NSR; ++s) {
+        Real& qq = qn[s * Np];
+        const Real rs = r[s];
+        qq = mul_add(bdt * rs, MJI, qq);
+        r[s] = rs * ka;
+      }
+      if (Phys::HAS_ADVECTION && advection) {
+        const Real Ht = qn[Np * 2] + qn[Np * 3];
+        qn[0] = Ht * uu;
+        qn[Np] = Ht * vv;
+      }
     }
-  } else if (!UPDATE && valid) {
-    Real rv[NSR];
-    Real* rr = sB + slot * BUF + NFN * NSR + n;
-#pragma unroll
-    for (int s = 0; s < NSR; ++s) rv[s] = rr[s * Np];
-    face_terms_at_node<DIM, NQ, NSR>(rv, sB + slot * BUF, sV + slot * NFN, n, NOVID);
-#pragma unroll
-    for (int s = 0; s < NSR; ++s) rr[s * Np] = rv[s];
   }
-  // 5. update: Qout = Q + ((rkb*dt)*rhs)*MJI, rhs *= rka, in LDS, by the
-  //    thread that holds the node's MJI (which, unless the face terms were
-  //    scattered, first takes its own face terms).  Shallow water with
-  //    `advection` keeps the velocity: u = Hu / (h + b) before the update,
-  //    Hu = (h + b) u after it (shallow_water.jl:274-297).
-  if (UPDATE && valid) {
-    // prepared arrays hold no MJI: the reference's is 1 ./ MJ (IEEE division)
-    // (FP32: refined estimate)
-    if constexpr (PREP) MJI = one_over(MJ);
-    const Real bdt = (Real)(rkb * dt);
-    const Real ka = (Real)rka;
-    Real* qn = sQ + slot * NS * Np + n;
-    Real uu = 0, vv = 0;
-    if (Phys::HAS_ADVECTION && advection) {
-      const Real Ht = qn[Np * 2] + qn[Np * 3];
-      uu = qn[0] / Ht;
-      vv = qn[Np] / Ht;
-    }
-    Real rv[NSR];
+  if (valid) {
 #pragma unroll
-    for (int s = 0; s < NSR; ++s) rv[s] = sB[slot * BUF + NFN * NSR + s * Np + n];
-    if (!scatter) face_terms_at_node<DIM, NQ, NSR>(rv, sB + slot * BUF, sV + slot * NFN, n, NOVID);
-#pragma unroll
-    for (int s = 0; s < NSR; ++s) {
-      Real& qq = qn[s * Np];
-      const Real rs = rv[s];
-      qq = mul_add(bdt * rs, MJI, qq);
-      sB[slot * BUF + NFN * NSR + s * Np + n] = rs * ka;
-    }
-    if (Phys::HAS_ADVECTION && advection) {
-      const Real Ht = qn[Np * 2] + qn[Np * 3];
-      qn[0] = Ht * uu;
-      qn[Np] = Ht * vv;
-    }
+    for (int s = 0; s < NSR; ++s) sB[slot * BUF + NFN * NSR + s * Np + n] = r[s];
   }
   lds_barrier();
   // 6. the block's results leave LDS in storage order: consecutive lanes
@@ -947,16 +998,16 @@ __device__ __forceinline__ void stage_body(
     for (int i = t; i < nv * NS * Np; i += NT) __builtin_nontemporal_store(sQ[i], &qo[i]);
   }
   {
-    Real* re = rhs + (size_t)NS * Np * (size_t)e0;
+    Real* ro = rhs + (size_t)NS * Np * (size_t)e0;
     for (int i = t; i < nv * NSR * Np; i += NT) {
-      const int sl = i / (NSR * Np), j = i - sl * (NSR * Np);
-      __builtin_nontemporal_store(sB[sl * BUF + NFN * NSR + j], &re[(size_t)sl * NS * Np + j]);
+      const int sl = EPW == 1 ? 0 : i / (NSR * Np), j = i - sl * (NSR * Np);
+      __builtin_nontemporal_store(sB[sl * BUF + NFN * NSR + j], &ro[sl * (NS * Np) + j]);
     }
   }
 }
 
 template <class Phys, int NQ, int EPW, bool WIDE, int PF, bool PM_LDS, bool MFMA = false>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, WIDE>::NT)) void stage_kernel(
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, WIDE>::NT), (stage_waves<Phys, NQ>())) void stage_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ vgeo, const double* __restrict__ sgeo,
     const double* __restrict__ D, int64_t nreal, int64_t ntotal,
@@ -976,7 +1027,7 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, WIDE>::NT)) void stage_ker
 // The fused stage over the prepared arrays (see Prepared): the same
 // arithmetic and order, fewer bytes.
 template <class Phys, int NQ, int EPW, int PF, bool MFMA = false>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void stage_prep_kernel(
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT), (stage_waves<Phys, NQ>())) void stage_prep_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ pvgeo, const double* __restrict__ psgeo,
     const int32_t* __restrict__ pface, const double* __restrict__ D, int64_t nreal,

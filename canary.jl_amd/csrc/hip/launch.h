@@ -64,12 +64,9 @@ inline int walk_back(const void* qin, const void* qout) {
 template <class Phys, int NQ, int EPW, bool MFMA = false>
 void launch_stage(int64_t nb, const KArgs& a) {
   // measured on 3D N=4 (32^3): one prefetched face item per thread, the
-  // nodal pressure cached in LDS, workgroup sized by the volume nodes.
-  // 3D N=6 prefetches none: 90 VGPRs instead of 112 make it five waves per
-  // SIMD, so three of its 384-lane workgroups fit a CU instead of two
-  // (23^3: 298 -> 266 us per stage; every other N is slower without it)
+  // nodal pressure cached in LDS, workgroup sized by the volume nodes
   constexpr bool WIDE = false;
-  constexpr int PF = (Phys::DIM == 3 && NQ == 7) ? 0 : 1;
+  constexpr int PF = 1;
   constexpr bool PM_LDS = true;
   constexpr int NT = FusedCfg<Phys, NQ, EPW, WIDE>::NT;
   const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
@@ -81,7 +78,7 @@ void launch_stage(int64_t nb, const KArgs& a) {
 
 template <class Phys, int NQ, int EPW, bool MFMA = false>
 void launch_stage_prep(int64_t nb, const KArgs& a) {
-  constexpr int PF = (Phys::DIM == 3 && NQ == 7) ? 0 : 1;  // as launch_stage
+  constexpr int PF = 1;  // as launch_stage
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
   const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
   stage_prep_kernel<Phys, NQ, EPW, PF, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(

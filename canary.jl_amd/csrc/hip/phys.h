@@ -94,6 +94,7 @@ __device__ __attribute__((noinline)) inline double pow_by_exp_log(double x, doub
 }
 
 struct FastOps {
+  static constexpr bool EXACT = false;
   __device__ static double recip(double x) {
     double r = __builtin_amdgcn_rcp(x);
     double e = fma(-x, r, 1.0);
@@ -135,6 +136,7 @@ struct FastOps {
 // gets the same bits (with kappa's table, when the host has made one, the
 // same bits come from the cheaper fast phase).
 struct ExactOps {
+  static constexpr bool EXACT = true;
   __device__ static double recip(double x) { return 1 / x; }
   __device__ static double powk(double x, const PhysParams& p) {
     return crpow::pow_cr_tab(x, p.kappa, p.ktab);
@@ -145,6 +147,7 @@ struct ExactOps {
 template <class Ops>
 struct Euler3DT {
   using Real = double;
+  static constexpr bool EXACT = Ops::EXACT;  // the reference's evaluation order
   static constexpr int DIM = 3, NS = 5, NSR = 5, NVGEO = 14, NSGEO = 5;
   static constexpr int iMJ = 9, iMJI = 10;
   static constexpr bool HAS_P = true, B_FROM_M = false, HAS_ADVECTION = false;
@@ -190,22 +193,33 @@ struct Euler3DT {
     const double nx = n[0], ny = n[1], nz = n[2];
     const double UM = qM[U], VM = qM[V], WM = qM[W], rM = qM[RHO], EM = qM[E];
     const double UP = qP[U], VP = qP[V], WP = qP[W], rP = qP[RHO], EP = qP[E];
-    const double rMi = Ops::recip(rM);
-    const double frMx = UM, fUMx = rMi * UM * UM + PM, fVMx = rMi * VM * UM, fWMx = rMi * WM * UM, fEMx = rMi * UM * EM;
-    const double frMy = VM, fUMy = rMi * UM * VM, fVMy = rMi * VM * VM + PM, fWMy = rMi * WM * VM, fEMy = rMi * VM * EM;
-    const double frMz = WM, fUMz = rMi * UM * WM, fVMz = rMi * VM * WM, fWMz = rMi * WM * WM + PM, fEMz = rMi * WM * EM;
-    const double rPi = Ops::recip(rP);
-    const double frPx = UP, fUPx = rPi * UP * UP + PP, fVPx = rPi * VP * UP, fWPx = rPi * WP * UP, fEPx = rPi * UP * EP;
-    const double frPy = VP, fUPy = rPi * UP * VP, fVPy = rPi * VP * VP + PP, fWPy = rPi * WP * VP, fEPy = rPi * VP * EP;
-    const double frPz = WP, fUPz = rPi * UP * WP, fVPz = rPi * VP * WP, fWPz = rPi * WP * WP + PP, fEPz = rPi * WP * EP;
+    // one component at a time: the flux components of all five live at once
+    // cost ten more registers than the stage has to spare
+    const double rMi = Ops::recip(rM), rPi = Ops::recip(rP);
     const double lM = rMi * fabs(nx * UM + ny * VM + nz * WM) + sqrt(rMi * p.gamma * PM);
     const double lP = rPi * fabs(nx * UP + ny * VP + nz * WP) + sqrt(rPi * p.gamma * PP);
     const double l = jmax(lM, lP);
-    out[RHO] = sMJ * ((nx * (frMx + frPx) + ny * (frMy + frPy) + nz * (frMz + frPz) - l * (rP - rM)) / 2);
-    out[U] = sMJ * ((nx * (fUMx + fUPx) + ny * (fUMy + fUPy) + nz * (fUMz + fUPz) - l * (UP - UM)) / 2);
-    out[V] = sMJ * ((nx * (fVMx + fVPx) + ny * (fVMy + fVPy) + nz * (fVMz + fVPz) - l * (VP - VM)) / 2);
-    out[W] = sMJ * ((nx * (fWMx + fWPx) + ny * (fWMy + fWPy) + nz * (fWMz + fWPz) - l * (WP - WM)) / 2);
-    out[E] = sMJ * ((nx * (fEMx + fEPx) + ny * (fEMy + fEPy) + nz * (fEMz + fEPz) - l * (EP - EM)) / 2);
+    out[RHO] = sMJ * ((nx * (UM + UP) + ny * (VM + VP) + nz * (WM + WP) - l * (rP - rM)) / 2);
+    {
+      const double Mx = rMi * UM * UM + PM, My = rMi * UM * VM, Mz = rMi * UM * WM;
+      const double Px = rPi * UP * UP + PP, Py = rPi * UP * VP, Pz = rPi * UP * WP;
+      out[U] = sMJ * ((nx * (Mx + Px) + ny * (My + Py) + nz * (Mz + Pz) - l * (UP - UM)) / 2);
+    }
+    {
+      const double Mx = rMi * VM * UM, My = rMi * VM * VM + PM, Mz = rMi * VM * WM;
+      const double Px = rPi * VP * UP, Py = rPi * VP * VP + PP, Pz = rPi * VP * WP;
+      out[V] = sMJ * ((nx * (Mx + Px) + ny * (My + Py) + nz * (Mz + Pz) - l * (VP - VM)) / 2);
+    }
+    {
+      const double Mx = rMi * WM * UM, My = rMi * WM * VM, Mz = rMi * WM * WM + PM;
+      const double Px = rPi * WP * UP, Py = rPi * WP * VP, Pz = rPi * WP * WP + PP;
+      out[W] = sMJ * ((nx * (Mx + Px) + ny * (My + Py) + nz * (Mz + Pz) - l * (WP - WM)) / 2);
+    }
+    {
+      const double Mx = rMi * UM * EM, My = rMi * VM * EM, Mz = rMi * WM * EM;
+      const double Px = rPi * UP * EP, Py = rPi * VP * EP, Pz = rPi * WP * EP;
+      out[E] = sMJ * ((nx * (Mx + Px) + ny * (My + Py) + nz * (Mz + Pz) - l * (EP - EM)) / 2);
+    }
   }
 };
 
