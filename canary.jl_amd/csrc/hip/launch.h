@@ -76,8 +76,27 @@ void launch_stage(int64_t nb, const KArgs& a) {
       a.dt, order, a.phys, a.advection);
 }
 
+// Elements per workgroup of the contracted prepared 2D stage on large meshes:
+// as many as 256 lanes hold.  Wider blocks read and write with fewer ragged
+// ends and hold more of their neighbours; they pay where a stage moves more
+// than the memory-side cache holds (from two million nodes on, 360 MB), below
+// that the latency of a workgroup counts.  us per step, narrow against wide:
+// 512^2 N=4 Euler 1,130 / 1,078, 500^2 N=2 421 / 402, 420^2 N=3 446 / 433,
+// 250^2 N=7 595 / 577, shallow water 400^2 N=4 640 / 627, 250^2 N=7 532 / 522;
+// smaller: 260^2 N=2 130 / 136, 150^2 N=7 220 / 225, 10 x 10 (50 stages) 241 /
+// 267.  Kept narrow: N=1 (600^2: 271 / 292), the exact order, which needs more
+// registers (200^2 N=7 454 / 473), 3D (32^3 N=4 1,051 / 1,085), and the
+// reference arrays (shallow water 250^2 N=2 140 / 145).
+template <class Phys, int NQ, int EPW>
+constexpr int large_prep_epw() {
+  constexpr int Np = Shape<Phys, NQ>::Np;
+  return Phys::DIM == 2 && !Phys::EXACT && NQ > 2 && 256 / Np > EPW ? 256 / Np : EPW;
+}
+constexpr int64_t kLargePrepNodes = 2000000;
+
 template <class Phys, int NQ, int EPW, bool MFMA = false>
-void launch_stage_prep(int64_t nb, const KArgs& a) {
+void launch_stage_prep(const KArgs& a) {
+  const int64_t nb = (a.nreal + EPW - 1) / EPW;
   constexpr int PF = 1;  // as launch_stage
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
   const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
@@ -90,8 +109,14 @@ void launch_stage_prep(int64_t nb, const KArgs& a) {
 // The prepared arrays hold no node heights: equation sets whose pressure
 // needs them have no prepared stage.
 template <class Phys, int NQ, int EPW, bool MFMA = false>
-void launch_stage_prep_if(int64_t nb, const KArgs& a) {
-  if constexpr (!NeedsY<Phys>::value) launch_stage_prep<Phys, NQ, EPW, MFMA>(nb, a);
+void launch_stage_prep_if(const KArgs& a) {
+  if constexpr (!NeedsY<Phys>::value) {
+    constexpr int BIG = large_prep_epw<Phys, NQ, EPW>();
+    if constexpr (BIG > EPW)
+      if (a.nreal * Shape<Phys, NQ>::Np >= kLargePrepNodes)
+        return launch_stage_prep<Phys, NQ, BIG, MFMA>(a);
+    launch_stage_prep<Phys, NQ, EPW, MFMA>(a);
+  }
 }
 
 template <class Phys, int NQ, int EPW, bool MFMA>
@@ -147,7 +172,7 @@ int launch(int op, const KArgs& a) {
     if (op == OP_STAGE)
       launch_stage<Phys, NQ, EPW, MFMA>(nb, a);
     else if (op == OP_STAGE_PREP && !NeedsY<Phys>::value)
-      launch_stage_prep_if<Phys, NQ, EPW, MFMA>(nb, a);
+      launch_stage_prep_if<Phys, NQ, EPW, MFMA>(a);
     else if (op == OP_VOLUME)
       launch_volume<Phys, NQ, EPW, MFMA>(nb, a);
     else if (op == OP_FACE_UPDATE || op == OP_FACE || op == OP_UPDATE) {
@@ -179,7 +204,7 @@ int launch(int op, const KArgs& a) {
         break;
       case OP_STAGE_PREP:
         if (NeedsY<Phys>::value) return 2 /*CANARY_ERR_UNSUPPORTED*/;
-        launch_stage_prep_if<Phys, NQ, EPW>(nb, a);
+        launch_stage_prep_if<Phys, NQ, EPW>(a);
         break;
       case OP_FACE_UPDATE:
         launch_face_update<Phys, NQ, EPW>(nb, a);

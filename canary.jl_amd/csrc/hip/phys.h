@@ -230,6 +230,7 @@ struct Euler3DFma : Euler3DT<FastOps> {};
 template <class Ops>
 struct Euler2DT {
   using Real = double;
+  static constexpr bool EXACT = Ops::EXACT;  // the reference's evaluation order
   static constexpr int DIM = 2, NS = 4, NSR = 4, NVGEO = 8, NSGEO = 4;
   static constexpr int iMJ = 4, iMJI = 5;
   static constexpr bool HAS_P = true, B_FROM_M = false, HAS_ADVECTION = false;
@@ -297,6 +298,7 @@ struct Euler2DFma : Euler2DT<FastOps> {};
 template <class Ops>
 struct Euler2DTET {
   using Real = double;
+  static constexpr bool EXACT = Ops::EXACT;  // the reference's evaluation order
   static constexpr int DIM = 2, NS = 4, NSR = 4, NVGEO = 8, NSGEO = 4;
   static constexpr int iMJ = 4, iMJI = 5, iY = 7;
   static constexpr bool HAS_P = true, B_FROM_M = false, HAS_ADVECTION = false, NEEDS_Y = true;
@@ -384,6 +386,7 @@ __device__ __forceinline__ typename Phys::Real pressure_at(const typename Phys::
 // Q = (H u, H v, h, b); b (bathymetry / still depth) has no tendency.
 struct SWE2D {
   using Real = double;
+  static constexpr bool EXACT = true;  // the reference's evaluation order
   static constexpr int DIM = 2, NS = 4, NSR = 3, NVGEO = 8, NSGEO = 4;
   static constexpr int iMJ = 4, iMJI = 5;
   // B_FROM_M: the reference face kernel reads the P-side b from element eM
@@ -452,7 +455,9 @@ struct SWE2D {
 // every unit that instantiates a template with the same arguments, and the
 // host launch stub is one symbol; with one type for both units, launches
 // from the contracted unit ran the exact-order unit's code.
-struct SWE2DFma : SWE2D {};
+struct SWE2DFma : SWE2D {
+  static constexpr bool EXACT = false;
+};
 
 // --------------------------------------------- shallow water, FP32 variant
 // The fluxes of SWE2D evaluated in FP32 (batched FP32 ensembles), in the form
@@ -468,6 +473,7 @@ struct SWE2DFma : SWE2D {};
 // register against 64 bits: h 8% closer, the momenta the same on average.
 struct SWE2DF32 {
   using Real = float;
+  static constexpr bool EXACT = false;
   static constexpr int DIM = 2, NS = 4, NSR = 3, NVGEO = 8, NSGEO = 4;
   static constexpr int iMJ = 4, iMJI = 5;
   static constexpr bool HAS_P = false, B_FROM_M = true, HAS_ADVECTION = true;
