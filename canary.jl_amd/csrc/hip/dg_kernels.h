@@ -649,7 +649,8 @@ __global__ __launch_bounds__(256) void update_kernel(double* __restrict__ rhs,
 //   4. face fluxes -> LDS, taken by each node's thread in ascending face order;
 //   5. update: Qout = Q + ((rkb*dt)*rhs)*MJI, rhs *= rka, to LDS;
 //   6. the block's Qout and rhs written out in storage order.
-template <class Phys, int NQ, int EPW, bool WIDE>
+// RES: room for rhs beside the face terms.
+template <class Phys, int NQ, int EPW, bool WIDE, bool RES = true>
 struct FusedCfg {
   // vidM of each face node fits a byte up to Np = 255, else a short
   using VidT = typename std::conditional<(Shape<Phys, NQ>::Np < 256), uint8_t, uint16_t>::type;
@@ -660,8 +661,9 @@ struct FusedCfg {
   static constexpr int NFACEIT = round64(EPW * S::NFN);
   static constexpr int NT = WIDE && NFACEIT > NVOL ? NFACEIT : NVOL;
   static constexpr int FLUX = S::Np;                       // per state, one direction
-  static constexpr int FACE = S::NFN + S::Np;               // face terms + rhs per state
-  static constexpr int BUF = (FLUX > FACE ? FLUX : FACE) * Phys::NSR;
+  static constexpr int FACE = S::NFN + (RES ? S::Np : 0);   // face terms + rhs per state
+  static constexpr int FLUX_ = RES ? FLUX : 0;              // (late_rhs: no fluxes)
+  static constexpr int BUF = (FLUX_ > FACE ? FLUX_ : FACE) * Phys::NSR;
   // LDS carve-up (bytes, each piece 16-byte aligned)
   static constexpr int a16(int b) { return (b + 15) / 16 * 16; }
   static constexpr int OFF_D = 0;
@@ -700,6 +702,17 @@ constexpr int stage_waves() {  // waves a SIMD must hold
   return Phys::DIM == 3 && NQ == 7 ? 5 : 1;
 }
 
+// facerhs! alone at these 3D orders reads rhs after the face terms and leaves
+// its results in Q's place, which nothing reads any more by then: without
+// rhs beside the face terms a third less LDS, so more workgroups fit a CU.  us
+// per launch, exact / contracted: N=1 70^3 203 / 154 -> 190 / 149, N=2 53^3 240 /
+// 185 -> 223 / 177, N=6 23^3 185 / 138 -> 181 / 126, N=7 20^3 161 / 121 -> 153 / 115;
+// N = 3, 4, 5 are level or 2-3% faster with rhs read at the start, as 2D is.
+template <class Phys, int NQ>
+constexpr bool late_rhs() {
+  return Phys::DIM == 3 && (NQ <= 3 || NQ >= 7);
+}
+
 // One fused stage of the EPW-element block starting at e0, computed by NT
 // threads (NT >= the volume nodes of the block).  `lds` holds
 // FusedCfg::LDS bytes.  PF: face items per thread whose loads are issued
@@ -720,7 +733,8 @@ __device__ __forceinline__ void stage_body(
     const int64_t* __restrict__ bndy, double rka, double rkb, double dt, const PhysParams& p,
     int advection = 0) {
   using S = Shape<Phys, NQ>;
-  using C = FusedCfg<Phys, NQ, EPW, false>;
+  constexpr bool LATE_R = !VOLUME && !UPDATE && late_rhs<Phys, NQ>();
+  using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
   using Real = typename Phys::Real;
   constexpr int Np = S::Np, DIM = S::DIM, NS = Phys::NS, NSR = Phys::NSR;
   constexpr int NV = PREP ? Prepared<Phys>::NV : Phys::NVGEO;
@@ -735,7 +749,7 @@ __device__ __forceinline__ void stage_body(
   constexpr bool LATE = VOLUME && gather_late<Phys, NQ>();
   constexpr bool N6 = stage_waves<Phys, NQ>() > 1;
   constexpr bool MAPS_LATE = LATE && !PREP && N6;
-  constexpr bool STAGE_R = !VOLUME || N6;  // rhs waits in LDS for the face terms
+  constexpr bool STAGE_R = (!VOLUME && !LATE_R) || (VOLUME && N6);  // rhs waits in LDS for the face terms
   constexpr int NSG = PREP ? Prepared<Phys>::NSG : Phys::NSGEO;
   constexpr bool SP = Phys::HAS_P && PM_LDS;
   constexpr int BUF = C::BUF;
@@ -750,6 +764,9 @@ __device__ __forceinline__ void stage_body(
   Real* sB = reinterpret_cast<Real*>(lds + C::OFF_B);  // [EPW][BUF]
   VidT* sV = reinterpret_cast<VidT*>(lds + C::OFF_V);  // [EPW][NFN]
   int* sFlag = reinterpret_cast<int*>(lds + C::OFF_F);  // a non-canonical M-side node seen
+
+  Real* sR = LATE_R ? sQ : sB + NFN * NSR;  // rhs results, RSTR words an element
+  constexpr int RSTR = LATE_R ? NS * Np : BUF;
 
   const int t = threadIdx.x;
   const int slot = EPW == 1 ? 0 : t / Np, n = t - slot * Np;
@@ -800,8 +817,10 @@ __device__ __forceinline__ void stage_body(
     MJ = vg[Np * Phys::iMJ];
   }
   const Real* re = rhs + (size_t)NS * Np * (size_t)e0 + (sl0 * NS * Np + nl);
+  if constexpr (!LATE_R) {
 #pragma unroll
-  for (int s = 0; s < NSR; ++s) r[s] = re[Np * s];
+    for (int s = 0; s < NSR; ++s) r[s] = re[Np * s];
+  }
   // maps checked as soon as they arrive and the P-side gathers issued
   // (unconditionally, as above: lanes without an item check the item
   // they loaded, e0's first face node, which some lane owns anyway)
@@ -936,6 +955,10 @@ __device__ __forceinline__ void stage_body(
     for (int s = 0; s < NSR; ++s) sB[sl * BUF + fi * NSR + s] = c[s];
   }
   if (!PREP && noncanon) *sFlag = 1;
+  if constexpr (LATE_R) {
+#pragma unroll
+    for (int s = 0; s < NSR; ++s) r[s] = re[Np * s];
+  }
   lds_barrier();
   // 5. each node's thread takes its own face terms in ascending face order
   //    (with the canonical face mask, always so over the prepared arrays, it
@@ -982,7 +1005,7 @@ __device__ __forceinline__ void stage_body(
   }
   if (valid) {
 #pragma unroll
-    for (int s = 0; s < NSR; ++s) sB[slot * BUF + NFN * NSR + s * Np + n] = r[s];
+    for (int s = 0; s < NSR; ++s) sR[slot * RSTR + s * Np + n] = r[s];
   }
   lds_barrier();
   // 6. the block's results leave LDS in storage order: consecutive lanes
@@ -1001,7 +1024,7 @@ __device__ __forceinline__ void stage_body(
     Real* ro = rhs + (size_t)NS * Np * (size_t)e0;
     for (int i = t; i < nv * NSR * Np; i += NT) {
       const int sl = EPW == 1 ? 0 : i / (NSR * Np), j = i - sl * (NSR * Np);
-      __builtin_nontemporal_store(sB[sl * BUF + NFN * NSR + j], &ro[sl * (NS * Np) + j]);
+      __builtin_nontemporal_store(sR[sl * RSTR + j], &ro[sl * (NS * Np) + j]);
     }
   }
 }
@@ -1055,7 +1078,7 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_ker
     const double* __restrict__ sgeo, int64_t nreal, int64_t ntotal,
     const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, BlockOrder order, PhysParams p) {
-  using C = FusedCfg<Phys, NQ, EPW, false>;
+  using C = FusedCfg<Phys, NQ, EPW, false, !late_rhs<Phys, NQ>()>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
