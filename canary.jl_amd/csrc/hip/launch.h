@@ -61,8 +61,36 @@ inline int walk_back(const void* qin, const void* qout) {
   return (uintptr_t)qin > (uintptr_t)qout ? 1 : 0;
 }
 
+// Elements per workgroup of a stage.
+//
+// Small 2D meshes (at most kSmallBlocks blocks, eight workgroups a CU) take
+// blocks of one wave: they wait for the latency of a workgroup, and one wave
+// has no other to wait for at its barriers.  us for 4 steps, default against
+// one wave: N=4 10 x 10 96 / 92, N=5 10 x 10 103 / 91, N=6 30 x 30 129 / 120,
+// shallow water 40 x 40 N=4 123 / 108, N=6 156 / 143, total energy 40 x 40 N=4 133 /
+// 116; above that size the default is ahead (N=5 50 x 50 149 / 161, N=6 170 / 174).
+// 3D N = 2 takes two elements, one wave, at every size: 20^3 103 / 88 us a step,
+// 36^3 451 / 428, 53^3 1,405 / 1,374, prepared exact 1,513 / 1,463 (its volume and
+// face kernels keep seven: facerhs 223 / 233).
+constexpr int64_t kSmallBlocks = 8 * 256;
+
+template <class Phys, int NQ, bool MFMA>
+constexpr int stage_epw() {
+  constexpr int Np = Shape<Phys, NQ>::Np;
+  return Phys::DIM == 3 && NQ == 3 && !MFMA ? 64 / Np : default_epw<Np>();
+}
+
+// 0: no narrower block than the default
+template <class Phys, int NQ>
+constexpr int small_epw() {
+  constexpr int Np = Shape<Phys, NQ>::Np;
+  constexpr int w = Np <= 64 ? 64 / Np : 0;
+  return Phys::DIM == 2 && w < default_epw<Np>() ? w : 0;
+}
+
 template <class Phys, int NQ, int EPW, bool MFMA = false>
-void launch_stage(int64_t nb, const KArgs& a) {
+void launch_stage(const KArgs& a) {
+  const int64_t nb = (a.nreal + EPW - 1) / EPW;
   // measured on 3D N=4 (32^3): one prefetched face item per thread, the
   // nodal pressure cached in LDS, workgroup sized by the volume nodes
   constexpr bool WIDE = false;
@@ -74,6 +102,14 @@ void launch_stage(int64_t nb, const KArgs& a) {
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.D, a.nreal, a.ntotal, a.vmapM, a.vmapP, a.bndy, a.rka, a.rkb,
       a.dt, order, a.phys, a.advection);
+}
+
+template <class Phys, int NQ, bool MFMA>
+void launch_stage_sized(const KArgs& a) {
+  constexpr int SMALL = small_epw<Phys, NQ>();
+  if constexpr (SMALL > 0)
+    if (a.nreal <= kSmallBlocks * SMALL) return launch_stage<Phys, NQ, SMALL, MFMA>(a);
+  launch_stage<Phys, NQ, stage_epw<Phys, NQ, MFMA>(), MFMA>(a);
 }
 
 // Elements per workgroup of the contracted prepared 2D stage on large meshes:
@@ -108,9 +144,13 @@ void launch_stage_prep(const KArgs& a) {
 
 // The prepared arrays hold no node heights: equation sets whose pressure
 // needs them have no prepared stage.
-template <class Phys, int NQ, int EPW, bool MFMA = false>
+template <class Phys, int NQ, bool MFMA = false>
 void launch_stage_prep_if(const KArgs& a) {
   if constexpr (!NeedsY<Phys>::value) {
+    constexpr int EPW = stage_epw<Phys, NQ, MFMA>();
+    constexpr int SMALL = small_epw<Phys, NQ>();
+    if constexpr (SMALL > 0)
+      if (a.nreal <= kSmallBlocks * SMALL) return launch_stage_prep<Phys, NQ, SMALL, MFMA>(a);
     constexpr int BIG = large_prep_epw<Phys, NQ, EPW>();
     if constexpr (BIG > EPW)
       if (a.nreal * Shape<Phys, NQ>::Np >= kLargePrepNodes)
@@ -170,9 +210,9 @@ int launch(int op, const KArgs& a) {
   const int64_t nb = (a.nreal + EPW - 1) / EPW;
   if constexpr (UNIT != UNIT_EXACT) {
     if (op == OP_STAGE)
-      launch_stage<Phys, NQ, EPW, MFMA>(nb, a);
+      launch_stage_sized<Phys, NQ, MFMA>(a);
     else if (op == OP_STAGE_PREP && !NeedsY<Phys>::value)
-      launch_stage_prep_if<Phys, NQ, EPW, MFMA>(a);
+      launch_stage_prep_if<Phys, NQ, MFMA>(a);
     else if (op == OP_VOLUME)
       launch_volume<Phys, NQ, EPW, MFMA>(nb, a);
     else if (op == OP_FACE_UPDATE || op == OP_FACE || op == OP_UPDATE) {
@@ -200,11 +240,11 @@ int launch(int op, const KArgs& a) {
         if (launch_update<Phys, NQ>(a)) return 1 /*CANARY_ERR_ARG*/;
         break;
       case OP_STAGE:
-        launch_stage<Phys, NQ, EPW>(nb, a);
+        launch_stage_sized<Phys, NQ, false>(a);
         break;
       case OP_STAGE_PREP:
         if (NeedsY<Phys>::value) return 2 /*CANARY_ERR_UNSUPPORTED*/;
-        launch_stage_prep_if<Phys, NQ, EPW>(a);
+        launch_stage_prep_if<Phys, NQ>(a);
         break;
       case OP_FACE_UPDATE:
         launch_face_update<Phys, NQ, EPW>(nb, a);
