@@ -92,7 +92,7 @@ __device__ __forceinline__ void solve_stage(char* lds, const canary_batch_solve&
 // per-thread face and LDS addressing live across iterations and costs
 // about 100 VGPRs in 3D; one entry per workgroup does not.)
 template <class Phys, int NQ, int EPW, bool PREP>
-__global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT)) void batched_kernel(
+__global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>())) void batched_kernel(
     const canary_batch_solve* __restrict__ solves, const canary_batch_item* __restrict__ items,
     int64_t nitems, BlockOrder order, int parity, double rka, double rkb,
     const crpow::KappaTable* __restrict__ ktabs, int nktab) {
@@ -117,10 +117,11 @@ __global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT)) void batched_kernel(
         p.ktab = ktabs + i;
         break;
       }
-  // 3D N=6 prefetches no face item (fewer VGPRs: a third 384-lane
-  // workgroup per CU), as the single-solve stage does
-  solve_stage<Phys, NQ, EPW, C::NT, (Phys::DIM == 3 && NQ == 7 && EPW == 1) ? 0 : 1, PREP>(
-      lds, sv, it.e0, parity, rka, rkb, p);
+  // one face item prefetched and five waves a SIMD at 3D N=6, as the
+  // single-solve stage.  Six N=6 bubbles of 8^3..13^3, us a step, no item
+  // prefetched against this: exact 1,129 / 960, contracted 903 / 775; prepared
+  // 1,036 / 980 and 820 / 743
+  solve_stage<Phys, NQ, EPW, C::NT, 1, PREP>(lds, sv, it.e0, parity, rka, rkb, p);
 }
 
 // ---------------------------------------------- every class in one launch

@@ -219,7 +219,7 @@ struct FaceItem {
   Real qP[Phys::NS];
   Real yP;  // height of the P node (equation sets whose pressure needs it)
   int64_t eP;
-  int64_t idM, idP, bcode;  // map and bc entries as loaded (face_load)
+  int64_t idM, idP, bcode;  // map and bc entries as loaded (face_load_maps)
   int vidM;  // -1: no contribution (an error was recorded)
   int vidP;
   int bc;
