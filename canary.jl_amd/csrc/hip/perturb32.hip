@@ -133,15 +133,17 @@ __device__ __forceinline__ int fmask(int f, int fn) {
   }
 }
 
-// expm1(kappa log1p(x)) by the device library, out of line: the path outside
-// the series' range.
-__device__ __attribute__((noinline)) float expm1_klog1p(float x, float kappa) {
-  return expm1f(kappa * log1pf(x));
+// expm1(kappa log1p(a / b)) by the device library, out of line: the path
+// outside the series' range.
+__device__ __attribute__((noinline)) float expm1_klog1p(float a, float b, float kappa) {
+  return expm1f(kappa * log1pf(a / b));
 }
 
+// (the estimated quotient is not finite where it does not hold: a background
+// above 2^126, where it would be zero, has an infinite P0)
 __device__ __forceinline__ float pprime(float P0, float rt0, float rtp, const P32Params& p) {
-  const float x = div32(rtp, rt0, __builtin_amdgcn_rcpf(rt0));
-  if (!(fabsf(x) <= p.xmax)) return P0 * expm1_klog1p(x, p.kappa);
+  const float x = div_est(rtp, rt0, __builtin_amdgcn_rcpf(rt0));
+  if (!(fabsf(x) <= p.xmax)) return P0 * expm1_klog1p(rtp, rt0, p.kappa);
   float a = p.c[kSeries - 1];
 #pragma unroll
   for (int i = kSeries - 2; i >= 0; --i) a = fmaf(a, x, p.c[i]);
@@ -431,10 +433,20 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
       UnM += nn[c] * qM[c];
       UnP += nn[c] * qPl[c];
     }
-    const float rMi = recip32(rM), rPi = recip32(rP);
-    const float unM = UnM * rMi, unP = UnP * rPi;
-    const float lM = fabsf(unM) + sqrt32(div32(p.gamma * (P0 + PpM), rM, rMi));
-    const float lP = fabsf(unP) + sqrt32(div32(p.gamma * (P0 + PpP), rP, rPi));
+    const float rMi = recip_est(rM), rPi = recip_est(rP);
+    float unM = UnM * rMi, unP = UnP * rPi;
+    const float gpM = p.gamma * (P0 + PpM), gpP = p.gamma * (P0 + PpP);
+    const float c2M = div_est(gpM, rM, rMi), c2P = div_est(gpP, rP, rPi);
+    float cM = sqrt_est(c2M), cP = sqrt_est(c2P);
+    // positive normal squares (class mask 0x100) are there for finite reciprocals alone
+    const bool ok = __builtin_amdgcn_classf(c2M, 0x100) & __builtin_amdgcn_classf(c2P, 0x100);
+    if (__builtin_expect(!ok, 0)) {
+      unM = UnM / rM;
+      unP = UnP / rP;
+      cM = sqrtf(gpM / rM);
+      cP = sqrtf(gpP / rP);
+    }
+    const float lM = fabsf(unM) + cM, lP = fabsf(unP) + cP;
     const float l = fmaxf(lM, lP);
     float nfM[NS], nfP[NS];
 #pragma unroll
@@ -475,7 +487,9 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
   // The node owner takes its own face terms, in ascending face order, and
   // updates; its results go to LDS and from there out in storage order.
   if (valid) {
-    const double MJI = FastOps::recip((double)MJg);  // the reference's MJI is 1 ./ MJ
+    // the reference's MJI is 1 ./ MJ; the estimate holds where it is a normal number
+    double MJI = FastOps::recip((double)MJg);
+    if (__builtin_expect(!__builtin_amdgcn_class(MJI, 0x108), 0)) MJI = 1.0 / (double)MJg;
     const int ni = n % NQ, nj = (n / NQ) % NQ, nk = DIM == 3 ? n / (NQ * NQ) : 0;
     const float* fc = L.B[slot];
 #pragma unroll

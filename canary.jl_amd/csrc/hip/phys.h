@@ -50,27 +50,46 @@ __device__ __forceinline__ double jmax(double a, double b) {
 }
 
 // ------------------------------------------------------------ FP32 arithmetic
-// 1 / x and a / b by the hardware estimate (within an ulp) and one Newton
-// step in fused multiply-adds: within an ulp, a third of the instructions of
-// the IEEE division, whose scaling steps serve operands near the ends of the
-// exponent range (densities, depths and rho*theta are not there).
-__device__ __forceinline__ float recip32(float x) {
+// 1 / x, a / b and sqrt(x) by the hardware estimate (within an ulp) and one
+// Newton step in fused multiply-adds: within an ulp, about half of the
+// instructions of the IEEE operations, whose scaling steps serve operands
+// near the ends of the exponent range.
+//
+// There (zero, infinity, subnormal numbers, x > 2^126, a quotient that
+// overflows) the steps give NaN or zero instead, so every use tests its values
+// with the predicates below and takes the IEEE operations where one fails, in
+// a branch that no lane enters in a state with ordinary depths and densities.
+// A dry or empty node then has the infinite speed that blows the solve up at
+// once, not a NaN that the larger of two speeds would drop.  One branch for
+// all operations of a face or a node: a branch each cost small launches up to
+// 5%.
+__device__ __forceinline__ float recip_est(float x) {
   const float r = __builtin_amdgcn_rcpf(x);
   return fmaf(fmaf(-x, r, 1.f), r, r);
 }
-// a / b, r the hardware estimate of 1 / b or recip32(b)
-__device__ __forceinline__ float div32(float a, float b, float r) {
+// r = recip_est(x) holds: a normal number (class mask 0x108).  The hardware
+// takes subnormal numbers for zero and gives zero for x > 2^126.
+__device__ __forceinline__ bool recip_ok(float r) { return __builtin_amdgcn_classf(r, 0x108); }
+// a / b, r = recip_est(b) or the hardware's; holds where it and r are finite
+__device__ __forceinline__ float div_est(float a, float b, float r) {
   const float q = a * r;
   return fmaf(fmaf(-b, q, a), r, q);
 }
-
-// sqrt(x): the hardware root (within an ulp) and one Newton step where x is a
-// positive normal number (class mask 0x100); 0, infinity and NaN as the
-// hardware gives them.
-__device__ __forceinline__ float sqrt32(float x) {
+__device__ __forceinline__ bool finite32(float x) { return fabsf(x) <= 0x1.fffffep127f; }
+// sqrt(x); holds unless x is a positive subnormal number (mask 0x80).  Zero,
+// infinity, NaN and negative numbers as the hardware gives them (mask 0x100:
+// positive normal).
+__device__ __forceinline__ float sqrt_est(float x) {
   const float s = __builtin_amdgcn_sqrtf(x);
   const float c = fmaf(fmaf(-s, s, x), 0.5f * __builtin_amdgcn_rsqf(x), s);
   return __builtin_amdgcn_classf(x, 0x100) ? c : s;
+}
+__device__ __forceinline__ bool sqrt_ok(float x) { return !__builtin_amdgcn_classf(x, 0x80); }
+
+__device__ __forceinline__ float recip32(float x) {
+  const float r = recip_est(x);
+  if (__builtin_expect(!recip_ok(r), 0)) return 1.f / x;
+  return r;
 }
 
 // ------------------------------------------------------- arithmetic policies
@@ -489,8 +508,12 @@ struct SWE2DF32 {
                                      const PhysParams& p, float F[DIM][NSR]) {
     const float g = (float)p.swe_g, dnl = (float)p.dnl;
     const float Uq = q[U], Vq = q[V], h = q[H], b = q[B];
-    const float Ht = h + b, r = recip32(Ht);
-    const float u = div32(Uq, Ht, r), v = div32(Vq, Ht, r);
+    const float Ht = h + b, r = recip_est(Ht);
+    float u = div_est(Uq, Ht, r), v = div_est(Vq, Ht, r);
+    if (__builtin_expect(!(recip_ok(r) && finite32(fabsf(u) + fabsf(v))), 0)) {
+      u = Uq / Ht;
+      v = Vq / Ht;
+    }
     const float hd = head(h, b, g, dnl);
     const float fUx = fmaf(Uq * u, dnl, hd), fUy = Uq * v * dnl, fVy = fmaf(Vq * v, dnl, hd);
 #pragma unroll
@@ -518,9 +541,22 @@ struct SWE2DF32 {
     const float hP = qP[H], bP = qP[B], UP = qP[U], VP = qP[V];
     const float HM = hM + bM, HP = hP + bP;
     const float UnM = fmaf(nx, UM, ny * VM), UnP = fmaf(nx, UP, ny * VP);
-    const float unM = div32(UnM, HM, recip32(HM)), unP = div32(UnP, HP, recip32(HP));
-    const float lM = fmaf(fabsf(unM) + sqrt32(g * HM), dnl, sqrt32(g * bM) * (1.f - dnl));
-    const float lP = fmaf(fabsf(unP) + sqrt32(g * HP), dnl, sqrt32(g * bP) * (1.f - dnl));
+    const float rM = recip_est(HM), rP = recip_est(HP);
+    const float gM = g * HM, gP = g * HP, g0M = g * bM, g0P = g * bP;
+    float unM = div_est(UnM, HM, rM), unP = div_est(UnP, HP, rP);
+    float cM = sqrt_est(gM), cP = sqrt_est(gP), c0M = sqrt_est(g0M), c0P = sqrt_est(g0P);
+    const bool ok = recip_ok(rM) & recip_ok(rP) & finite32(fabsf(unM) + fabsf(unP)) &
+                    sqrt_ok(gM) & sqrt_ok(gP) & sqrt_ok(g0M) & sqrt_ok(g0P);
+    if (__builtin_expect(!ok, 0)) {
+      unM = UnM / HM;
+      unP = UnP / HP;
+      cM = sqrtf(gM);
+      cP = sqrtf(gP);
+      c0M = sqrtf(g0M);
+      c0P = sqrtf(g0P);
+    }
+    const float lM = fmaf(fabsf(unM) + cM, dnl, c0M * (1.f - dnl));
+    const float lP = fmaf(fabsf(unP) + cP, dnl, c0P * (1.f - dnl));
     const float l = fmaxf(lM, lP);
     const float hd = head(hM, bM, g, dnl) + head(hP, bP, g, dnl);
     const float fh = UnM + UnP;
