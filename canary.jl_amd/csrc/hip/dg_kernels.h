@@ -500,17 +500,59 @@ __device__ __forceinline__ void face_terms_at_node(Real* r, const Real* sC, cons
   }
 }
 
-// The same when vmapM is not the canonical face mask: the node owner looks
-// through every item's node in ascending order.
-template <int NFN, int NSR, class Real, class VidT>
-__device__ __forceinline__ void face_terms_by_search(Real* r, const Real* sC, const VidT* sV,
-                                                     int n) {
-#pragma unroll 1
-  for (int fi = 0; fi < NFN; ++fi)
-    if (sV[fi] == (VidT)n) {
+// The same for any vmapM, by the whole workgroup (EPW elements of which the
+// first nv are there, node n of element `slot` in r, items in sV and sC as
+// above with BUF words an element).  The items of each face pair leave their
+// number at their node in a table (tab: TSTR words of Real an element, free
+// until r is stored), and the node owner takes one term per pair, in
+// ascending order.  Where two items of a pair name one node, which no
+// numbering of a face does, the owners look through all items instead, which
+// is right for every map and several times the work.
+template <int DIM, int NQ, int EPW, int NT, int NSR, int BUF, int TSTR, class Real, class VidT>
+__device__ __forceinline__ void face_terms_any_map(Real* r, const Real* sB, const VidT* sV,
+                                                   Real* tab, int* sFlag, VidT novid, int nv,
+                                                   int slot, int n, bool valid) {
+  constexpr int Np = ipow(NQ, DIM), Nfp = ipow(NQ, DIM - 1), NFN = 2 * DIM * Nfp;
+  static_assert(sizeof(Real) * NSR >= sizeof(int) * DIM, "the table fits rhs's place");
+  auto table = [&](int sl) { return reinterpret_cast<int*>(tab + sl * TSTR); };
+  if (valid) {
 #pragma unroll
-      for (int s = 0; s < NSR; ++s) r[s] = r[s] - sC[fi * NSR + s];
+    for (int d = 0; d < DIM; ++d) table(slot)[d * Np + n] = -1;
+  }
+  lds_barrier();
+  for (int item = threadIdx.x; item < nv * NFN; item += NT) {
+    const int sl = EPW == 1 ? 0 : item / NFN, fi = item - sl * NFN;
+    if (sV[item] != novid) table(sl)[fi / (2 * Nfp) * Np + sV[item]] = fi;
+  }
+  lds_barrier();
+  for (int item = threadIdx.x; item < nv * NFN; item += NT) {
+    const int sl = EPW == 1 ? 0 : item / NFN, fi = item - sl * NFN;
+    if (sV[item] != novid && table(sl)[fi / (2 * Nfp) * Np + sV[item]] != fi) *sFlag = 2;
+  }
+  int fi[DIM];
+  if (valid) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) fi[d] = table(slot)[d * Np + n];
+  }
+  lds_barrier();  // the table is read (r may take its place) and checked
+  if (valid) {
+    const Real* sC = sB + slot * BUF;
+    if (*sFlag == 2) {
+#pragma unroll 1
+      for (int k = 0; k < NFN; ++k)
+        if (sV[slot * NFN + k] == (VidT)n) {
+#pragma unroll
+          for (int s = 0; s < NSR; ++s) r[s] = r[s] - sC[k * NSR + s];
+        }
+    } else {
+#pragma unroll
+      for (int d = 0; d < DIM; ++d)
+        if (fi[d] >= 0) {
+#pragma unroll
+          for (int s = 0; s < NSR; ++s) r[s] = r[s] - sC[fi[d] * NSR + s];
+        }
     }
+  }
 }
 
 // ================================================================ kernels
@@ -962,18 +1004,44 @@ __device__ __forceinline__ void stage_body(
   lds_barrier();
   // 5. each node's thread takes its own face terms in ascending face order
   //    (with the canonical face mask, always so over the prepared arrays, it
-  //    finds them from its indices; over the reference arrays, in a workgroup
-  //    with any other vmapM, it looks through the items' nodes), then updates.
+  //    finds them from its indices; over the reference arrays, a workgroup
+  //    with any other vmapM makes a table), then updates.
   //    Shallow water with `advection` keeps the velocity: u = Hu / (h + b)
   //    before the update, Hu = (h + b) u after it (shallow_water.jl:274-297).
+  bool any_map = false;
+  if constexpr (!PREP) {
+    any_map = __builtin_amdgcn_readfirstlane(*sFlag) != 0;
+    if (any_map) {
+      const int nv = nreal - e0 < EPW ? (int)(nreal - e0) : EPW;
+      if constexpr (STAGE_R) {
+        Real x[NSR];
+        Real* const xs = sB + slot * BUF + NFN * NSR + n;
+        if (valid) {
+#pragma unroll
+          for (int s = 0; s < NSR; ++s) x[s] = xs[s * Np];
+        }
+        lds_barrier();  // the table takes rhs's place
+        face_terms_any_map<DIM, NQ, EPW, NT, NSR, BUF, RSTR>(x, sB, sV, sR, sFlag, NOVID, nv,
+                                                             slot, n, valid);
+        if (valid) {
+#pragma unroll
+          for (int s = 0; s < NSR; ++s) xs[s * Np] = x[s];
+        }
+        // back through LDS, not kept in registers: live over this branch it
+        // would cost every launch eight of them
+        asm volatile("" ::: "memory");
+      } else {
+        face_terms_any_map<DIM, NQ, EPW, NT, NSR, BUF, RSTR>(r, sB, sV, sR, sFlag, NOVID, nv,
+                                                             slot, n, valid);
+      }
+    }
+  }
   if (valid) {
     if constexpr (STAGE_R) {
 #pragma unroll
       for (int s = 0; s < NSR; ++s) r[s] = sB[slot * BUF + NFN * NSR + s * Np + n];
     }
-    if (!PREP && *sFlag != 0)
-      face_terms_by_search<NFN, NSR>(r, sB + slot * BUF, sV + slot * NFN, n);
-    else
+    if (!any_map)
       face_terms_at_node<DIM, NQ, NSR>(r, sB + slot * BUF, sV + slot * NFN, n, NOVID);
     if constexpr (UPDATE) {
       // prepared arrays hold no MJI: the reference's is 1 ./ MJ (IEEE division;
