@@ -744,11 +744,10 @@ constexpr int stage_waves() {  // waves a SIMD must hold
   return Phys::DIM == 3 && NQ == 7 ? 5 : 1;
 }
 
-// facerhs! alone at these 3D orders reads rhs after the face terms and leaves
-// its results in Q's place, which nothing reads any more by then: without
-// rhs beside the face terms a third less LDS, so more workgroups fit a CU.  us
-// per launch, exact / contracted: N=1 70^3 203 / 154 -> 190 / 149, N=2 53^3 240 /
-// 185 -> 223 / 177, N=6 23^3 185 / 138 -> 181 / 126, N=7 20^3 161 / 121 -> 153 / 115;
+// facerhs! alone at these 3D orders may read rhs after the face terms and
+// leave its results in Q's place, which nothing reads any more by then: without
+// rhs beside the face terms a fifth (N=1) to a third (N=6, 7) less LDS, so more
+// workgroups fit a CU (late_rhs_pays in launch.h has the line).
 // N = 3, 4, 5 are level or 2-3% faster with rhs read at the start, as 2D is.
 template <class Phys, int NQ>
 constexpr bool late_rhs() {
@@ -763,9 +762,10 @@ constexpr bool late_rhs() {
 // VOLUME = false leaves the volume term out (face terms + update only: the
 // opt-in facerhs_update, after a separate volumerhs); vgeo is then read for
 // MJI alone and D is not read.  UPDATE = false (with VOLUME = false) is
-// facerhs! alone: rhs -= face terms, Q untouched, neither vgeo nor Qout read.
+// facerhs! alone: rhs -= face terms, Q untouched, neither vgeo nor Qout read;
+// LATE_R: rhs read after the face terms (late_rhs).
 template <class Phys, int NQ, int EPW, int NT, int PF, bool PM_LDS, bool VOLUME = true,
-          bool UPDATE = true, bool PREP = false, bool MFMA = false>
+          bool UPDATE = true, bool PREP = false, bool MFMA = false, bool LATE_R = false>
 __device__ __forceinline__ void stage_body(
     char* __restrict__ lds, typename Phys::Real* __restrict__ rhs,
     const typename Phys::Real* __restrict__ Qin, typename Phys::Real* __restrict__ Qout,
@@ -775,7 +775,7 @@ __device__ __forceinline__ void stage_body(
     const int64_t* __restrict__ bndy, double rka, double rkb, double dt, const PhysParams& p,
     int advection = 0) {
   using S = Shape<Phys, NQ>;
-  constexpr bool LATE_R = !VOLUME && !UPDATE && late_rhs<Phys, NQ>();
+  static_assert(!LATE_R || (!VOLUME && !UPDATE), "facerhs! alone");
   using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
   using Real = typename Phys::Real;
   constexpr int Np = S::Np, DIM = S::DIM, NS = Phys::NS, NSR = Phys::NSR;
@@ -1140,20 +1140,20 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT), (stage_waves<
 // the M side, non-temporal rhs stores) and the same bits.  vgeo is read only
 // by equation sets whose pressure needs the node height (else it may be
 // null).
-template <class Phys, int NQ, int EPW>
+template <class Phys, int NQ, int EPW, bool LATE_R>
 __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_kernel(
     double* __restrict__ rhs, const double* __restrict__ Q, const double* __restrict__ vgeo,
     const double* __restrict__ sgeo, int64_t nreal, int64_t ntotal,
     const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, BlockOrder order, PhysParams p) {
-  using C = FusedCfg<Phys, NQ, EPW, false, !late_rhs<Phys, NQ>()>;
+  using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, 1, true, false, false>(lds, rhs, Q, nullptr, vgeo, sgeo,
-                                                          nullptr, e0, nreal, ntotal, vmapM,
-                                                          vmapP, bndy, 0.0, 0.0, 0.0, p);
+  stage_body<Phys, NQ, EPW, C::NT, 1, true, false, false, false, false, LATE_R>(
+      lds, rhs, Q, nullptr, vgeo, sgeo, nullptr, e0, nreal, ntotal, vmapM, vmapP, bndy, 0.0, 0.0,
+      0.0, p);
 }
 
 // facerhs! + updatesolution! of one stage in one pass (the volume term was

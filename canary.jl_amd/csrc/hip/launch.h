@@ -168,13 +168,35 @@ void launch_volume(int64_t nb, const KArgs& a) {
       a.phys);
 }
 
+// facerhs! reads rhs late (see late_rhs) where its workgroups do not all fit the
+// 256 CUs' LDS at once with rhs read at the start.  Where they do, the smaller
+// LDS gains nothing and the later load is waited for.  us for five stages of
+// volumerhs! + facerhs! + updatesolution!, at the start / late, exact and
+// contracted: N=1 27^3 (2,461 workgroups, 3,072 fit) 156 / 167 and 139 / 150,
+// 33^3 235 / 228 and 205 / 199, 63^3 1,379 / 1,330 and 1,170 / 1,152; N=2 18^3 (833 of
+// 1,280) 161 / 166 and 141 / 147, 22^3 215 / 206 and 185 / 174, 53^3 2,526 / 2,452 and
+// 2,217 / 2,201; N=6 8^3 (512 of 768) 161 / 164 and 150 / 151, 12^3 355 / 345 and 305 /
+// 287; N=7 8^3 (512 of 512) 177 / 177 and 152 / 153, 11^3 376 / 357 and 336 / 318.
 template <class Phys, int NQ, int EPW>
-void launch_face(int64_t nb, const KArgs& a) {
+bool late_rhs_pays(int64_t nb) {
+  constexpr int64_t fit = 256 * (160 * 1024 / FusedCfg<Phys, NQ, EPW, false>::LDS);
+  return nb > fit;
+}
+
+template <class Phys, int NQ, int EPW, bool LATE_R>
+void launch_face_form(int64_t nb, const KArgs& a) {
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
   const BlockOrder order = block_order(nb, inplace_direction());
-  face_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
+  face_kernel<Phys, NQ, EPW, LATE_R><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, (const double*)a.sgeo, a.nreal,
       a.ntotal, a.vmapM, a.vmapP, a.bndy, order, a.phys);
+}
+
+template <class Phys, int NQ, int EPW>
+void launch_face(int64_t nb, const KArgs& a) {
+  if constexpr (late_rhs<Phys, NQ>())
+    if (late_rhs_pays<Phys, NQ, EPW>(nb)) return launch_face_form<Phys, NQ, EPW, true>(nb, a);
+  launch_face_form<Phys, NQ, EPW, false>(nb, a);
 }
 
 // Nonzero: the grid would not fit a launch.
