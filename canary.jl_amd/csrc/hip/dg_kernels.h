@@ -103,7 +103,8 @@ __device__ __forceinline__ void split_id(int64_t id1, int64_t& elem, int& node) 
 // way).  The blocks past the last whole round of runs, and a launch of fewer
 // than 16 runs per XCD, are split into contiguous pieces: such a mesh is in
 // flight nearly as a whole, and the longer pieces only keep more neighbours
-// together (one rank's 4,096 elements: 38.6 us against 39.3).
+// together (one rank's 4,096 elements: 38.6 us against 39.3).  `deal` false:
+// pieces alone (inplace_order in launch.h).
 //
 // A launch has 8*chunk workgroups and the map is one to one on them; the
 // blocks beyond the mesh leave at once.  The host works out the order, the
@@ -123,10 +124,10 @@ struct BlockOrder {
   uint32_t last;   // 8*chunk - 1 when walked backwards, else 0
 };
 
-inline BlockOrder block_order(int64_t nblocks, int reverse) {
+inline BlockOrder block_order(int64_t nblocks, int reverse, bool deal = true) {
   BlockOrder o;
   o.chunk = (uint32_t)((nblocks + 7) / 8);
-  o.dealt = o.chunk < 16 * kXcdRun ? 0 : o.chunk / kXcdRun * kXcdRun;
+  o.dealt = !deal || o.chunk < 16 * kXcdRun ? 0 : o.chunk / kXcdRun * kXcdRun;
   o.last = reverse ? 8 * o.chunk - 1 : 0;
   return o;
 }

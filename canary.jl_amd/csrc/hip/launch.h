@@ -55,6 +55,27 @@ inline int inplace_direction() {
   return (int)(n.fetch_add(1, std::memory_order_relaxed) & 1u);
 }
 
+// Block order of the in-place kernels.  A stage of them passes over the mesh
+// several times.  Where its arrays nearly fit the 256 MB memory-side cache (210
+// MB of them), a contiguous piece per XCD keeps each element on one XCD, and in
+// its L2, through all passes; above that the runs of block_order are ahead.
+// us for five stages of the three calls, in runs / in pieces: Euler 2D N=2 258^2
+// (99 MB) 321 / 307, N=3 274^2 (183 MB) contracted 394 / 376, N=7 137^2 (159 MB)
+// 420 / 404, total energy N=2 365^2 (198 MB) 514 / 492, shallow water N=7 137^2 320 /
+// 308; N=1 548^2 (230 MB) 598 / 613, shallow water 552 / 576.
+// facerhs_update reads and writes a second Q: N=2 258^2 485 / 464 us for two
+// steps, N=3 274^2 (221 MB) 664 / 698.
+constexpr int64_t kInplaceCache = 210000000;
+
+template <class Phys, int NQ>
+BlockOrder inplace_order(int64_t nblocks, const KArgs& a, bool second_q = false) {
+  using S = Shape<Phys, NQ>;
+  constexpr int DIM = Phys::DIM;
+  constexpr int64_t bytes = 8 * (S::Np * (Phys::NS + Phys::NSR + DIM * DIM + 2) + S::NFN * (DIM + 3));
+  const int64_t all = a.nreal * (bytes + (second_q ? 8 * S::Np * Phys::NS : 0));
+  return block_order(nblocks, inplace_direction(), all > kInplaceCache);
+}
+
 // Element order of a ping-pong stage: the two Q buffers swap roles every
 // stage, so their address order alternates and so does the direction.
 inline int walk_back(const void* qin, const void* qout) {
@@ -162,7 +183,7 @@ void launch_stage_prep_if(const KArgs& a) {
 template <class Phys, int NQ, int EPW, bool MFMA>
 void launch_volume(int64_t nb, const KArgs& a) {
   constexpr int NT = VolumeCfg<Phys, NQ, EPW>::NT;
-  const BlockOrder order = block_order(nb, inplace_direction());
+  const BlockOrder order = inplace_order<Phys, NQ>(nb, a);
   volume_kernel<Phys, NQ, EPW, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, a.D, a.nreal, order,
       a.phys);
@@ -186,7 +207,7 @@ bool late_rhs_pays(int64_t nb) {
 template <class Phys, int NQ, int EPW, bool LATE_R>
 void launch_face_form(int64_t nb, const KArgs& a) {
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
-  const BlockOrder order = block_order(nb, inplace_direction());
+  const BlockOrder order = inplace_order<Phys, NQ>(nb, a);
   face_kernel<Phys, NQ, EPW, LATE_R><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, (const double*)a.sgeo, a.nreal,
       a.ntotal, a.vmapM, a.vmapP, a.bndy, order, a.phys);
@@ -205,7 +226,7 @@ int launch_update(const KArgs& a) {
   const int64_t total = a.nreal * Shape<Phys, NQ>::Np;
   const int64_t nb = (total + 255) / 256;
   if (8 * ((nb + 7) / 8) > 0x7fffffffLL) return 1;
-  const BlockOrder order = block_order(nb, inplace_direction());
+  const BlockOrder order = inplace_order<Phys, NQ>(nb, a);
   update_kernel<Phys, NQ><<<dim3((unsigned)(8 * order.chunk)), dim3(256), 0, a.stream>>>(
       (double*)a.rhs, (double*)a.Qout, (const double*)a.vgeo, a.nreal, a.rka, a.rkb, a.dt,
       a.advection, order);
@@ -215,7 +236,7 @@ int launch_update(const KArgs& a) {
 template <class Phys, int NQ, int EPW>
 void launch_face_update(int64_t nb, const KArgs& a) {
   constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
-  const BlockOrder order = block_order(nb, inplace_direction());
+  const BlockOrder order = inplace_order<Phys, NQ>(nb, a, true);
   face_update_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.nreal, a.ntotal, a.vmapM, a.vmapP, a.bndy, a.rka, a.rkb, a.dt,
