@@ -90,6 +90,10 @@ inline int walk_back(const void* qin, const void* qout) {
 // one wave: N=4 10 x 10 96 / 92, N=5 10 x 10 103 / 91, N=6 30 x 30 129 / 120,
 // shallow water 40 x 40 N=4 123 / 108, N=6 156 / 143, total energy 40 x 40 N=4 133 /
 // 116; above that size the default is ahead (N=5 50 x 50 149 / 161, N=6 170 / 174).
+// Not where a SIMD would get more of these waves than a CU gets workgroups of
+// the default: it is then one round of workgroups longer (2 steps at N=6, shallow
+// water: 32 x 32, 1 and 1, default / one wave 64 / 61; 35 x 35, 1 and 2, 65 / 67; 36 x 36, 2
+// and 2, 73 / 67; N=5 33 x 33, 1 and 2, 63 / 68).
 // 3D N = 2 takes two elements, one wave, at every size: 20^3 103 / 88 us a step,
 // 36^3 451 / 428, 53^3 1,405 / 1,374, prepared exact 1,513 / 1,463 (its volume and
 // face kernels keep seven: facerhs 223 / 233).
@@ -107,6 +111,14 @@ constexpr int small_epw() {
   constexpr int Np = Shape<Phys, NQ>::Np;
   constexpr int w = Np <= 64 ? 64 / Np : 0;
   return Phys::DIM == 2 && w < default_epw<Np>() ? w : 0;
+}
+
+inline bool one_wave_blocks(int64_t nreal, int small, int epw) {
+  auto rounds = [&](int e, int per_round) {
+    const int64_t nb = (nreal + e - 1) / e;
+    return (nb + per_round - 1) / per_round;
+  };
+  return nreal <= kSmallBlocks * small && rounds(small, 4 * 256) <= rounds(epw, 256);
 }
 
 template <class Phys, int NQ, int EPW, bool MFMA = false>
@@ -128,9 +140,10 @@ void launch_stage(const KArgs& a) {
 template <class Phys, int NQ, bool MFMA>
 void launch_stage_sized(const KArgs& a) {
   constexpr int SMALL = small_epw<Phys, NQ>();
+  constexpr int EPW = stage_epw<Phys, NQ, MFMA>();
   if constexpr (SMALL > 0)
-    if (a.nreal <= kSmallBlocks * SMALL) return launch_stage<Phys, NQ, SMALL, MFMA>(a);
-  launch_stage<Phys, NQ, stage_epw<Phys, NQ, MFMA>(), MFMA>(a);
+    if (one_wave_blocks(a.nreal, SMALL, EPW)) return launch_stage<Phys, NQ, SMALL, MFMA>(a);
+  launch_stage<Phys, NQ, EPW, MFMA>(a);
 }
 
 // Elements per workgroup of the contracted prepared 2D stage on large meshes:
@@ -171,7 +184,7 @@ void launch_stage_prep_if(const KArgs& a) {
     constexpr int EPW = stage_epw<Phys, NQ, MFMA>();
     constexpr int SMALL = small_epw<Phys, NQ>();
     if constexpr (SMALL > 0)
-      if (a.nreal <= kSmallBlocks * SMALL) return launch_stage_prep<Phys, NQ, SMALL, MFMA>(a);
+      if (one_wave_blocks(a.nreal, SMALL, EPW)) return launch_stage_prep<Phys, NQ, SMALL, MFMA>(a);
     constexpr int BIG = large_prep_epw<Phys, NQ, EPW>();
     if constexpr (BIG > EPW)
       if (a.nreal * Shape<Phys, NQ>::Np >= kLargePrepNodes)
