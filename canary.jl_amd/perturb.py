@@ -79,31 +79,34 @@ class Perturb32:
             raise _lib.CanaryError(rc, "perturb32 (face %d, element %d, value %d)"
                                    % (info[1], info[2], info[3]))
 
-    def stage(self, rka, rkb, dt):
-        s = self.s
-        fn = lib().canary_stage_perturb_mixed if self.mixed else lib().canary_stage_perturb32
-        rc = fn(s.dim, s.N, _ptr(self.rhs), _ptr(self.q), _ptr(self.q2), _ptr(self.bg32),
-                _ptr(self.vg), _ptr(self.sg), _ptr(self.nbr), _ptr(self.D),
-                s.nelem, float(rka), float(rkb), float(dt), C.byref(s.phys), self._st())
-        check(rc, "perturb stage")
-        self.q, self.q2 = self.q2, self.q
-
-    def run(self, dt, nsteps):
-        """nsteps LSRK54 steps.  The stages of one call share their arguments
-        (small meshes wait for the host: 9.3 us a stage when each stage made
-        its own)."""
-        A, B, _ = rk_coefs()
+    def _stage_call(self):
+        """A function of (rka, rkb, dt) that runs one stage.  Its other
+        arguments are made here, once for all stages of a run (small meshes
+        wait for the host: 9.3 us a stage when each stage made its own)."""
         s = self.s
         fn = lib().canary_stage_perturb_mixed if self.mixed else lib().canary_stage_perturb32
         rhs, bg, vg, sg, nbr, D = (t.data_ptr() for t in (self.rhs, self.bg32, self.vg, self.sg,
                                                           self.nbr, self.D))
-        phys, st, dt = C.byref(s.phys), self._st(), float(dt)
+        phys, st = C.byref(s.phys), self._st()
+
+        def call(rka, rkb, dt):
+            rc = fn(s.dim, s.N, rhs, self.q.data_ptr(), self.q2.data_ptr(), bg, vg, sg, nbr, D,
+                    s.nelem, rka, rkb, dt, phys, st)
+            check(rc, "perturb stage")
+            self.q, self.q2 = self.q2, self.q
+
+        return call
+
+    def stage(self, rka, rkb, dt):
+        self._stage_call()(float(rka), float(rkb), float(dt))
+
+    def run(self, dt, nsteps):
+        """nsteps LSRK54 steps."""
+        A, B, _ = rk_coefs()
+        call, dt = self._stage_call(), float(dt)
         for _ in range(nsteps):
             for k in range(5):
-                rc = fn(s.dim, s.N, rhs, self.q.data_ptr(), self.q2.data_ptr(), bg, vg, sg, nbr, D,
-                        s.nelem, A[(k + 1) % 5], B[k], dt, phys, st)
-                check(rc, "perturb stage")
-                self.q, self.q2 = self.q2, self.q
+                call(A[(k + 1) % 5], B[k], dt)
 
     def full_state(self):
         s = self.s
