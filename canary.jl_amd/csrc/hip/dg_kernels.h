@@ -693,13 +693,16 @@ __global__ __launch_bounds__(256) void update_kernel(double* __restrict__ rhs,
 //   5. update: Qout = Q + ((rkb*dt)*rhs)*MJI, rhs *= rka, to LDS;
 //   6. the block's Qout and rhs written out in storage order.
 // RES: room for rhs beside the face terms.
-template <class Phys, int NQ, int EPW, bool RES = true>
+template <class Phys, int NQ, int EPW, bool WIDE, bool RES = true>
 struct FusedCfg {
   // vidM of each face node fits a byte up to Np = 255, else a short
   using VidT = typename std::conditional<(Shape<Phys, NQ>::Np < 256), uint8_t, uint16_t>::type;
   using S = Shape<Phys, NQ>;
   using Real = typename Phys::Real;
-  static constexpr int NT = round64(EPW * S::Np);
+  // WIDE: enough threads for every face item of the workgroup in one round
+  static constexpr int NVOL = round64(EPW * S::Np);
+  static constexpr int NFACEIT = round64(EPW * S::NFN);
+  static constexpr int NT = WIDE && NFACEIT > NVOL ? NFACEIT : NVOL;
   static constexpr int FLUX = S::Np;                       // per state, one direction
   static constexpr int FACE = S::NFN + (RES ? S::Np : 0);   // face terms + rhs per state
   static constexpr int FLUX_ = RES ? FLUX : 0;              // (late_rhs: no fluxes)
@@ -754,15 +757,16 @@ constexpr bool late_rhs() {
 
 // One fused stage of the EPW-element block starting at e0, computed by NT
 // threads (NT >= the volume nodes of the block).  `lds` holds
-// FusedCfg::LDS bytes.  Each thread's first face item is loaded with its node's
-// arrays (the rest, where there are more items than threads, afterwards).
+// FusedCfg::LDS bytes.  PF: face items per thread whose loads are issued
+// before the volume work (the rest are handled afterwards); PM_LDS: keep
+// the nodal pressure in LDS for the M side of the faces (else recompute it).
 // VOLUME = false leaves the volume term out (face terms + update only: the
 // opt-in facerhs_update, after a separate volumerhs); vgeo is then read for
 // MJI alone and D is not read.  UPDATE = false (with VOLUME = false) is
 // facerhs! alone: rhs -= face terms, Q untouched, neither vgeo nor Qout read;
 // LATE_R: rhs read after the face terms (late_rhs).
-template <class Phys, int NQ, int EPW, int NT, bool VOLUME = true, bool UPDATE = true,
-          bool PREP = false, bool MFMA = false, bool LATE_R = false>
+template <class Phys, int NQ, int EPW, int NT, int PF, bool PM_LDS, bool VOLUME = true,
+          bool UPDATE = true, bool PREP = false, bool MFMA = false, bool LATE_R = false>
 __device__ __forceinline__ void stage_body(
     char* __restrict__ lds, typename Phys::Real* __restrict__ rhs,
     const typename Phys::Real* __restrict__ Qin, typename Phys::Real* __restrict__ Qout,
@@ -773,21 +777,24 @@ __device__ __forceinline__ void stage_body(
     int advection = 0) {
   using S = Shape<Phys, NQ>;
   static_assert(!LATE_R || (!VOLUME && !UPDATE), "facerhs! alone");
-  using C = FusedCfg<Phys, NQ, EPW, !LATE_R>;
+  using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
   using Real = typename Phys::Real;
   constexpr int Np = S::Np, DIM = S::DIM, NS = Phys::NS, NSR = Phys::NSR;
   constexpr int NV = PREP ? Prepared<Phys>::NV : Phys::NVGEO;
   constexpr int NFN = S::NFN, Nfp = S::Nfp;
+  constexpr int KF = (EPW * NFN + NT - 1) / NT;
   static_assert(!PREP || (VOLUME && UPDATE), "prepared arrays: the whole stage only");
-  static_assert(!NeedsY<Phys>::value || !PREP,
-                "a pressure that needs y: the reference arrays hold it");
+  static_assert(!NeedsY<Phys>::value || (PM_LDS && !PREP),
+                "a pressure that needs y: M side from LDS, reference arrays (which hold y)");
   // prepared arrays: psgeo in `sgeo`, the face codes in `vmapP`'s place
   const int32_t* __restrict__ pface = reinterpret_cast<const int32_t*>(vmapP);
+  constexpr int KP = PF < KF ? PF : KF;
   constexpr bool LATE = VOLUME && gather_late<Phys, NQ>();
   constexpr bool N6 = stage_waves<Phys, NQ>() > 1;
   constexpr bool MAPS_LATE = LATE && !PREP && N6;
   constexpr bool STAGE_R = (!VOLUME && !LATE_R) || (VOLUME && N6);  // rhs waits in LDS for the face terms
   constexpr int NSG = PREP ? Prepared<Phys>::NSG : Phys::NSGEO;
+  constexpr bool SP = Phys::HAS_P && PM_LDS;
   constexpr int BUF = C::BUF;
   using VidT = typename C::VidT;
   constexpr VidT NOVID = (VidT)~(VidT)0;
@@ -809,21 +816,27 @@ __device__ __forceinline__ void stage_body(
   const bool valid = EPW == 1 ? t < Np : slot < EPW && e0 + slot < nreal;
 
   // 1. issue the loads of the block before any of them is used: the face
-  //    item's maps and bc (item t), D, the node's Q, metric terms and
+  //    items' maps and bc (t, t + NT, ...), D, the node's Q, metric terms and
   //    rhs -- one memory round trip instead of one per kind.  The loads are
   //    unconditional (lanes without work read in-bounds element e0, node 0,
   //    and ignore it): a load under a branch makes every later wait count
   //    for the path without it, i.e. wait for everything.
-  FaceItem<Phys> fit;
-  int fsl = EPW == 1 ? 0 : t / NFN;
-  const bool fval = t < EPW * NFN && (EPW == 1 || e0 + fsl < nreal);
-  fsl = fval ? fsl : 0;
-  const int ffi = fval ? t - fsl * NFN : 0;
-  if constexpr (PREP)
-    face_load_code<Phys, NQ>(fit, pface, e0 + fsl, ffi);
-  else if constexpr (!MAPS_LATE)
-    face_load_maps<Phys, NQ>(fit, vmapM, vmapP, bndy, e0 + fsl, ffi);
-  if constexpr (!LATE) face_load_geo<Phys, NQ, NSG>(fit, sgeo, e0 + fsl, ffi);
+  FaceItem<Phys> fit[KP > 0 ? KP : 1];  // KP = 0: every face item after the volume work
+  bool fval[KP > 0 ? KP : 1];
+  int fsl[KP > 0 ? KP : 1], ffi[KP > 0 ? KP : 1];
+#pragma unroll
+  for (int k = 0; k < KP; ++k) {
+    const int item = t + k * NT;
+    fsl[k] = EPW == 1 ? 0 : item / NFN;
+    fval[k] = item < EPW * NFN && (EPW == 1 || e0 + fsl[k] < nreal);
+    fsl[k] = fval[k] ? fsl[k] : 0;
+    ffi[k] = fval[k] ? item - fsl[k] * NFN : 0;
+    if constexpr (PREP)
+      face_load_code<Phys, NQ>(fit[k], pface, e0 + fsl[k], ffi[k]);
+    else if constexpr (!MAPS_LATE)
+      face_load_maps<Phys, NQ>(fit[k], vmapM, vmapP, bndy, e0 + fsl[k], ffi[k]);
+    if constexpr (!LATE) face_load_geo<Phys, NQ, NSG>(fit[k], sgeo, e0 + fsl[k], ffi[k]);
+  }
   double dval = 0.0;
   if constexpr (VOLUME) dval = D[t < NQ * NQ ? t : 0];
   // keep the map loads ahead of the node loads: waiting for the maps then
@@ -855,12 +868,16 @@ __device__ __forceinline__ void stage_body(
   // (unconditionally, as above: lanes without an item check the item
   // they loaded, e0's first face node, which some lane owns anyway)
   auto gather = [&]() {
-    if constexpr (LATE && !MAPS_LATE) face_load_geo<Phys, NQ, NSG>(fit, sgeo, e0 + fsl, ffi);
-    if constexpr (PREP)
-      face_decode_resolve<Phys, NQ>(fit, e0 + fsl, ffi, ntotal);
-    else
-      face_resolve<Phys, NQ>(fit, e0 + fsl, ffi, ntotal);
-    face_gather_any<Phys, NQ>(fit, Qin, vgeo, fval, e0);
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+      if constexpr (LATE && !MAPS_LATE)
+        face_load_geo<Phys, NQ, NSG>(fit[k], sgeo, e0 + fsl[k], ffi[k]);
+      if constexpr (PREP)
+        face_decode_resolve<Phys, NQ>(fit[k], e0 + fsl[k], ffi[k], ntotal);
+      else
+        face_resolve<Phys, NQ>(fit[k], e0 + fsl[k], ffi[k], ntotal);
+      face_gather_any<Phys, NQ>(fit[k], Qin, vgeo, fval[k], e0);
+    }
   };
   if constexpr (!LATE) gather();
 
@@ -872,7 +889,7 @@ __device__ __forceinline__ void stage_body(
 #pragma unroll
     for (int s = 0; s < NS; ++s) sQ[slot * NS * Np + s * Np + n] = q[s];
     const Real P = Phys::HAS_P ? pressure_at<Phys>(q, ynode, p) : Real(0);
-    if (Phys::HAS_P) sP[slot * Np + n] = P;
+    if (SP) sP[slot * Np + n] = P;
     if constexpr (VOLUME) {
       Phys::volume_flux(q, P, met, MJ, p, Fv);
       Phys::source(q, MJ, p, r);
@@ -881,8 +898,11 @@ __device__ __forceinline__ void stage_body(
   if constexpr (LATE) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (MAPS_LATE) {
-      face_load_maps<Phys, NQ>(fit, vmapM, vmapP, bndy, e0 + fsl, ffi);
-      face_load_geo<Phys, NQ, NSG>(fit, sgeo, e0 + fsl, ffi);
+#pragma unroll
+      for (int k = 0; k < KP; ++k) {
+        face_load_maps<Phys, NQ>(fit[k], vmapM, vmapP, bndy, e0 + fsl[k], ffi[k]);
+        face_load_geo<Phys, NQ, NSG>(fit[k], sgeo, e0 + fsl[k], ffi[k]);
+      }
     } else {
       gather();
     }
@@ -934,22 +954,31 @@ __device__ __forceinline__ void stage_body(
   }
   // 4. face fluxes: M side from LDS, P side gathered
   bool noncanon = false;  // an item whose M-side node is not the canonical one
-  auto pm_of = [&](int sl, int v) -> Real { return Phys::HAS_P ? sP[sl * Np + v] : Real(0); };
-  if (fval) {
-    auto qm_at = [&](int s, int v) { return sQ[fsl * NS * Np + s * Np + v]; };
-    auto pm_at = [&](int v, const Real*) { return pm_of(fsl, v); };
-    Real c[NSR];
-    const int vid = face_finish<Phys>(fit, p, qm_at, pm_at, c);
-    if constexpr (!PREP) noncanon |= vid >= 0 && vid != canon_vid<DIM, NQ>(ffi / Nfp, ffi % Nfp);
-    sV[fsl * NFN + ffi] = vid < 0 ? NOVID : (VidT)vid;
+  auto pm_of = [&](int sl, int v, const Real* qm) -> Real {
+    if (!Phys::HAS_P) return Real(0);
+    if constexpr (SP)
+      return sP[sl * Np + v];
+    else
+      return Phys::pressure(qm, p);  // (a pressure that needs y always has SP)
+  };
 #pragma unroll
-    for (int s = 0; s < NSR; ++s) sB[fsl * BUF + ffi * NSR + s] = c[s];
+  for (int k = 0; k < KP; ++k) {
+    if (!fval[k]) continue;
+    const int sl = fsl[k], fi = ffi[k];
+    auto qm_at = [&](int s, int v) { return sQ[sl * NS * Np + s * Np + v]; };
+    auto pm_at = [&](int v, const Real* qm) { return pm_of(sl, v, qm); };
+    Real c[NSR];
+    const int vid = face_finish<Phys>(fit[k], p, qm_at, pm_at, c);
+    if constexpr (!PREP) noncanon |= vid >= 0 && vid != canon_vid<DIM, NQ>(fi / Nfp, fi % Nfp);
+    sV[sl * NFN + fi] = vid < 0 ? NOVID : (VidT)vid;
+#pragma unroll
+    for (int s = 0; s < NSR; ++s) sB[sl * BUF + fi * NSR + s] = c[s];
   }
-  for (int item = t + NT; item < EPW * NFN; item += NT) {
+  for (int item = t + KP * NT; item < EPW * NFN; item += NT) {
     const int sl = EPW == 1 ? 0 : item / NFN, fi = item - sl * NFN;
     if (EPW > 1 && e0 + sl >= nreal) continue;
     auto qm_at = [&](int s, int v) { return sQ[sl * NS * Np + s * Np + v]; };
-    auto pm_at = [&](int v, const Real*) { return pm_of(sl, v); };
+    auto pm_at = [&](int v, const Real* qm) { return pm_of(sl, v, qm); };
     Real c[NSR];
     int vid;
     if constexpr (PREP) {
@@ -1069,39 +1098,39 @@ __device__ __forceinline__ void stage_body(
   }
 }
 
-template <class Phys, int NQ, int EPW, bool MFMA = false>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>())) void stage_kernel(
+template <class Phys, int NQ, int EPW, bool WIDE, int PF, bool PM_LDS, bool MFMA = false>
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, WIDE>::NT), (stage_waves<Phys, NQ>())) void stage_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ vgeo, const double* __restrict__ sgeo,
     const double* __restrict__ D, int64_t nreal, int64_t ntotal,
     const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, double rka, double rkb, double dt,
     BlockOrder order, PhysParams p, int advection) {
-  using C = FusedCfg<Phys, NQ, EPW>;
+  using C = FusedCfg<Phys, NQ, EPW, WIDE>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, true, true, false, MFMA>(
+  stage_body<Phys, NQ, EPW, C::NT, PF, PM_LDS, true, true, false, MFMA>(
       lds, rhs, Qin, Qout, vgeo, sgeo, D, e0, nreal, ntotal, vmapM, vmapP, bndy, rka, rkb, dt, p,
       advection);
 }
 
 // The fused stage over the prepared arrays (see Prepared): the same
 // arithmetic and order, fewer bytes.
-template <class Phys, int NQ, int EPW, bool MFMA = false>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>())) void stage_prep_kernel(
+template <class Phys, int NQ, int EPW, int PF, bool MFMA = false>
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT), (stage_waves<Phys, NQ>())) void stage_prep_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ pvgeo, const double* __restrict__ psgeo,
     const int32_t* __restrict__ pface, const double* __restrict__ D, int64_t nreal,
     int64_t ntotal, double rka, double rkb, double dt, BlockOrder order, PhysParams p,
     int advection) {
-  using C = FusedCfg<Phys, NQ, EPW>;
+  using C = FusedCfg<Phys, NQ, EPW, false>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, true, true, true, MFMA>(
+  stage_body<Phys, NQ, EPW, C::NT, PF, true, true, true, true, MFMA>(
       lds, rhs, Qin, Qout, pvgeo, psgeo, D, e0, nreal, ntotal, nullptr,
       reinterpret_cast<const int64_t*>(pface), nullptr, rka, rkb, dt, p, advection);
 }
@@ -1113,17 +1142,17 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, N
 // by equation sets whose pressure needs the node height (else it may be
 // null).
 template <class Phys, int NQ, int EPW, bool LATE_R>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT)) void face_kernel(
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_kernel(
     double* __restrict__ rhs, const double* __restrict__ Q, const double* __restrict__ vgeo,
     const double* __restrict__ sgeo, int64_t nreal, int64_t ntotal,
     const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, BlockOrder order, PhysParams p) {
-  using C = FusedCfg<Phys, NQ, EPW, !LATE_R>;
+  using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, false, false, false, false, LATE_R>(
+  stage_body<Phys, NQ, EPW, C::NT, 1, true, false, false, false, false, LATE_R>(
       lds, rhs, Q, nullptr, vgeo, sgeo, nullptr, e0, nreal, ntotal, vmapM, vmapP, bndy, 0.0, 0.0,
       0.0, p);
 }
@@ -1131,18 +1160,18 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT)) void face_kernel(
 // facerhs! + updatesolution! of one stage in one pass (the volume term was
 // added to rhs by volume_kernel before): Qin -> Qout, rhs in place.
 template <class Phys, int NQ, int EPW>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT)) void face_update_kernel(
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_update_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ vgeo, const double* __restrict__ sgeo, int64_t nreal,
     int64_t ntotal, const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, double rka, double rkb, double dt,
     BlockOrder order, PhysParams p, int advection) {
-  using C = FusedCfg<Phys, NQ, EPW>;
+  using C = FusedCfg<Phys, NQ, EPW, false>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, false>(lds, rhs, Qin, Qout, vgeo, sgeo, nullptr, e0,
+  stage_body<Phys, NQ, EPW, C::NT, 1, true, false>(lds, rhs, Qin, Qout, vgeo, sgeo, nullptr, e0,
                                                    nreal, ntotal, vmapM, vmapP, bndy, rka, rkb,
                                                    dt, p, advection);
 }
