@@ -25,8 +25,7 @@ constexpr int MAXT = 256;  // threads per workgroup ceiling for several elements
 // Candidate `WHICH` of elements per workgroup for (DIM, NQ): 0 = the most
 // elements that fit MAXT threads (one element, with as many threads as it
 // has nodes, when it alone exceeds MAXT: 3D N = 6, 7), 1 = about half of
-// that, 2 = the single-solve choice (first lane fill >= 90%).  0 = no such
-// candidate.
+// that, 2 = the first lane fill >= 90%.  0 = no such candidate.
 template <int DIM, int NQ, int WHICH>
 constexpr int epw_candidate() {
   constexpr int Np = ipow(NQ, DIM);
@@ -58,14 +57,14 @@ __device__ __forceinline__ PhysParams params_of(const canary_phys& c) {
 
 template <class Phys, int NQ, int EPW>
 struct BCfg {
-  using C = FusedCfg<Phys, NQ, EPW, false>;
+  using C = FusedCfg<Phys, NQ, EPW>;
   static constexpr int NT = C::NT;
 };
 
 // One stage of the block at e0 of solve sv, over the reference arrays or,
 // PREP, over the prepared ones (pvgeo / psgeo in vgeo / sgeo, the face codes
 // in pface; the Prepared layout of dg_kernels.h).
-template <class Phys, int NQ, int EPW, int NT, int PF, bool PREP>
+template <class Phys, int NQ, int EPW, int NT, bool PREP>
 __device__ __forceinline__ void solve_stage(char* lds, const canary_batch_solve& sv, int64_t e0,
                                             int parity, double rka, double rkb,
                                             const PhysParams& p) {
@@ -77,12 +76,12 @@ __device__ __forceinline__ void solve_stage(char* lds, const canary_batch_solve&
   const Real* sgeo = as_global((const Real*)sv.sgeo);
   const double* D = as_global(sv.D);
   if constexpr (PREP)
-    stage_body<Phys, NQ, EPW, NT, PF, true, true, true, true>(
+    stage_body<Phys, NQ, EPW, NT, true, true, true>(
         lds, rhs, qin, qout, vgeo, sgeo, D, e0, sv.nreal, sv.nelem_total, nullptr,
         reinterpret_cast<const int64_t*>(as_global(sv.pface)), nullptr, rka, rkb, sv.dt, p,
         sv.advection);
   else
-    stage_body<Phys, NQ, EPW, NT, PF, true>(
+    stage_body<Phys, NQ, EPW, NT>(
         lds, rhs, qin, qout, vgeo, sgeo, D, e0, sv.nreal, sv.nelem_total, as_global(sv.vmapM),
         as_global(sv.vmapP), as_global(sv.elemtobndy), rka, rkb, sv.dt, p, sv.advection);
 }
@@ -96,7 +95,7 @@ __global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>()
     const canary_batch_solve* __restrict__ solves, const canary_batch_item* __restrict__ items,
     int64_t nitems, BlockOrder order, int parity, double rka, double rkb,
     const crpow::KappaTable* __restrict__ ktabs, int nktab) {
-  using C = FusedCfg<Phys, NQ, EPW, false>;
+  using C = FusedCfg<Phys, NQ, EPW>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t w = stage_block(blockIdx.x, order);  // direction alternates per stage
   if (w >= nitems) return;
@@ -121,7 +120,7 @@ __global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>()
   // single-solve stage.  Six N=6 bubbles of 8^3..13^3, us a step, no item
   // prefetched against this: exact 1,129 / 960, contracted 903 / 775; prepared
   // 1,036 / 980 and 820 / 743
-  solve_stage<Phys, NQ, EPW, C::NT, 1, PREP>(lds, sv, it.e0, parity, rka, rkb, p);
+  solve_stage<Phys, NQ, EPW, C::NT, PREP>(lds, sv, it.e0, parity, rka, rkb, p);
 }
 
 // ---------------------------------------------- every class in one launch
@@ -137,7 +136,7 @@ constexpr bool fits_all() {
 template <class Phys, int NQ>
 constexpr int all_lds_nq() {
   if constexpr (fits_all<Phys, NQ>())
-    return FusedCfg<Phys, NQ, epw_candidate<Phys::DIM, NQ, 0>(), false>::LDS;
+    return FusedCfg<Phys, NQ, epw_candidate<Phys::DIM, NQ, 0>()>::LDS;
   else
     return 0;
 }
@@ -158,7 +157,7 @@ __device__ __forceinline__ void all_item(char* lds, const canary_batch_solve& sv
                                          double rkb, const PhysParams& p) {
   if constexpr (fits_all<Phys, NQ>()) {
     constexpr int E = epw_candidate<Phys::DIM, NQ, 0>();
-    solve_stage<Phys, NQ, E, MAXT, 1, PREP>(lds, sv, it.e0, parity, rka, rkb, p);
+    solve_stage<Phys, NQ, E, MAXT, PREP>(lds, sv, it.e0, parity, rka, rkb, p);
   }
 }
 

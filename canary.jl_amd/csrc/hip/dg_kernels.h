@@ -693,16 +693,13 @@ __global__ __launch_bounds__(256) void update_kernel(double* __restrict__ rhs,
 //   5. update: Qout = Q + ((rkb*dt)*rhs)*MJI, rhs *= rka, to LDS;
 //   6. the block's Qout and rhs written out in storage order.
 // RES: room for rhs beside the face terms.
-template <class Phys, int NQ, int EPW, bool WIDE, bool RES = true>
+template <class Phys, int NQ, int EPW, bool RES = true>
 struct FusedCfg {
   // vidM of each face node fits a byte up to Np = 255, else a short
   using VidT = typename std::conditional<(Shape<Phys, NQ>::Np < 256), uint8_t, uint16_t>::type;
   using S = Shape<Phys, NQ>;
   using Real = typename Phys::Real;
-  // WIDE: enough threads for every face item of the workgroup in one round
-  static constexpr int NVOL = round64(EPW * S::Np);
-  static constexpr int NFACEIT = round64(EPW * S::NFN);
-  static constexpr int NT = WIDE && NFACEIT > NVOL ? NFACEIT : NVOL;
+  static constexpr int NT = round64(EPW * S::Np);
   static constexpr int FLUX = S::Np;                       // per state, one direction
   static constexpr int FACE = S::NFN + (RES ? S::Np : 0);   // face terms + rhs per state
   static constexpr int FLUX_ = RES ? FLUX : 0;              // (late_rhs: no fluxes)
@@ -757,16 +754,15 @@ constexpr bool late_rhs() {
 
 // One fused stage of the EPW-element block starting at e0, computed by NT
 // threads (NT >= the volume nodes of the block).  `lds` holds
-// FusedCfg::LDS bytes.  PF: face items per thread whose loads are issued
-// before the volume work (the rest are handled afterwards); PM_LDS: keep
-// the nodal pressure in LDS for the M side of the faces (else recompute it).
+// FusedCfg::LDS bytes.  Each thread's first face item is loaded with its node's
+// arrays (the rest, where there are more items than threads, afterwards).
 // VOLUME = false leaves the volume term out (face terms + update only: the
 // opt-in facerhs_update, after a separate volumerhs); vgeo is then read for
 // MJI alone and D is not read.  UPDATE = false (with VOLUME = false) is
 // facerhs! alone: rhs -= face terms, Q untouched, neither vgeo nor Qout read;
 // LATE_R: rhs read after the face terms (late_rhs).
-template <class Phys, int NQ, int EPW, int NT, int PF, bool PM_LDS, bool VOLUME = true,
-          bool UPDATE = true, bool PREP = false, bool MFMA = false, bool LATE_R = false>
+template <class Phys, int NQ, int EPW, int NT, bool VOLUME = true, bool UPDATE = true,
+          bool PREP = false, bool MFMA = false, bool LATE_R = false>
 __device__ __forceinline__ void stage_body(
     char* __restrict__ lds, typename Phys::Real* __restrict__ rhs,
     const typename Phys::Real* __restrict__ Qin, typename Phys::Real* __restrict__ Qout,
@@ -777,24 +773,25 @@ __device__ __forceinline__ void stage_body(
     int advection = 0) {
   using S = Shape<Phys, NQ>;
   static_assert(!LATE_R || (!VOLUME && !UPDATE), "facerhs! alone");
-  using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
+  using C = FusedCfg<Phys, NQ, EPW, !LATE_R>;
   using Real = typename Phys::Real;
   constexpr int Np = S::Np, DIM = S::DIM, NS = Phys::NS, NSR = Phys::NSR;
   constexpr int NV = PREP ? Prepared<Phys>::NV : Phys::NVGEO;
   constexpr int NFN = S::NFN, Nfp = S::Nfp;
-  constexpr int KF = (EPW * NFN + NT - 1) / NT;
   static_assert(!PREP || (VOLUME && UPDATE), "prepared arrays: the whole stage only");
-  static_assert(!NeedsY<Phys>::value || (PM_LDS && !PREP),
-                "a pressure that needs y: M side from LDS, reference arrays (which hold y)");
+  static_assert(!NeedsY<Phys>::value || !PREP,
+                "a pressure that needs y: the reference arrays hold it");
   // prepared arrays: psgeo in `sgeo`, the face codes in `vmapP`'s place
   const int32_t* __restrict__ pface = reinterpret_cast<const int32_t*>(vmapP);
-  constexpr int KP = PF < KF ? PF : KF;
+  // Face items per thread loaded with the node's arrays.  More than one costs
+  // registers.  The code over them stays loops of one: written straight out, the
+  // compiler moves the item's loads under `if (fval)` (10 x 10 loop 231.7 -> 235.4 us).
+  constexpr int KP = 1;
   constexpr bool LATE = VOLUME && gather_late<Phys, NQ>();
   constexpr bool N6 = stage_waves<Phys, NQ>() > 1;
   constexpr bool MAPS_LATE = LATE && !PREP && N6;
   constexpr bool STAGE_R = (!VOLUME && !LATE_R) || (VOLUME && N6);  // rhs waits in LDS for the face terms
   constexpr int NSG = PREP ? Prepared<Phys>::NSG : Phys::NSGEO;
-  constexpr bool SP = Phys::HAS_P && PM_LDS;
   constexpr int BUF = C::BUF;
   using VidT = typename C::VidT;
   constexpr VidT NOVID = (VidT)~(VidT)0;
@@ -821,9 +818,9 @@ __device__ __forceinline__ void stage_body(
   //    unconditional (lanes without work read in-bounds element e0, node 0,
   //    and ignore it): a load under a branch makes every later wait count
   //    for the path without it, i.e. wait for everything.
-  FaceItem<Phys> fit[KP > 0 ? KP : 1];  // KP = 0: every face item after the volume work
-  bool fval[KP > 0 ? KP : 1];
-  int fsl[KP > 0 ? KP : 1], ffi[KP > 0 ? KP : 1];
+  FaceItem<Phys> fit[KP];
+  bool fval[KP];
+  int fsl[KP], ffi[KP];
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
     const int item = t + k * NT;
@@ -889,7 +886,7 @@ __device__ __forceinline__ void stage_body(
 #pragma unroll
     for (int s = 0; s < NS; ++s) sQ[slot * NS * Np + s * Np + n] = q[s];
     const Real P = Phys::HAS_P ? pressure_at<Phys>(q, ynode, p) : Real(0);
-    if (SP) sP[slot * Np + n] = P;
+    if constexpr (Phys::HAS_P) sP[slot * Np + n] = P;
     if constexpr (VOLUME) {
       Phys::volume_flux(q, P, met, MJ, p, Fv);
       Phys::source(q, MJ, p, r);
@@ -955,11 +952,10 @@ __device__ __forceinline__ void stage_body(
   // 4. face fluxes: M side from LDS, P side gathered
   bool noncanon = false;  // an item whose M-side node is not the canonical one
   auto pm_of = [&](int sl, int v, const Real* qm) -> Real {
-    if (!Phys::HAS_P) return Real(0);
-    if constexpr (SP)
+    if constexpr (Phys::HAS_P)
       return sP[sl * Np + v];
     else
-      return Phys::pressure(qm, p);  // (a pressure that needs y always has SP)
+      return Phys::pressure(qm, p);
   };
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
@@ -1098,39 +1094,39 @@ __device__ __forceinline__ void stage_body(
   }
 }
 
-template <class Phys, int NQ, int EPW, bool WIDE, int PF, bool PM_LDS, bool MFMA = false>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, WIDE>::NT), (stage_waves<Phys, NQ>())) void stage_kernel(
+template <class Phys, int NQ, int EPW, bool MFMA = false>
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>())) void stage_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ vgeo, const double* __restrict__ sgeo,
     const double* __restrict__ D, int64_t nreal, int64_t ntotal,
     const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, double rka, double rkb, double dt,
     BlockOrder order, PhysParams p, int advection) {
-  using C = FusedCfg<Phys, NQ, EPW, WIDE>;
+  using C = FusedCfg<Phys, NQ, EPW>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, PF, PM_LDS, true, true, false, MFMA>(
+  stage_body<Phys, NQ, EPW, C::NT, true, true, false, MFMA>(
       lds, rhs, Qin, Qout, vgeo, sgeo, D, e0, nreal, ntotal, vmapM, vmapP, bndy, rka, rkb, dt, p,
       advection);
 }
 
 // The fused stage over the prepared arrays (see Prepared): the same
 // arithmetic and order, fewer bytes.
-template <class Phys, int NQ, int EPW, int PF, bool MFMA = false>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT), (stage_waves<Phys, NQ>())) void stage_prep_kernel(
+template <class Phys, int NQ, int EPW, bool MFMA = false>
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>())) void stage_prep_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ pvgeo, const double* __restrict__ psgeo,
     const int32_t* __restrict__ pface, const double* __restrict__ D, int64_t nreal,
     int64_t ntotal, double rka, double rkb, double dt, BlockOrder order, PhysParams p,
     int advection) {
-  using C = FusedCfg<Phys, NQ, EPW, false>;
+  using C = FusedCfg<Phys, NQ, EPW>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, PF, true, true, true, true, MFMA>(
+  stage_body<Phys, NQ, EPW, C::NT, true, true, true, MFMA>(
       lds, rhs, Qin, Qout, pvgeo, psgeo, D, e0, nreal, ntotal, nullptr,
       reinterpret_cast<const int64_t*>(pface), nullptr, rka, rkb, dt, p, advection);
 }
@@ -1142,17 +1138,17 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT), (stage_waves<
 // by equation sets whose pressure needs the node height (else it may be
 // null).
 template <class Phys, int NQ, int EPW, bool LATE_R>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_kernel(
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT)) void face_kernel(
     double* __restrict__ rhs, const double* __restrict__ Q, const double* __restrict__ vgeo,
     const double* __restrict__ sgeo, int64_t nreal, int64_t ntotal,
     const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, BlockOrder order, PhysParams p) {
-  using C = FusedCfg<Phys, NQ, EPW, false, !LATE_R>;
+  using C = FusedCfg<Phys, NQ, EPW, !LATE_R>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, 1, true, false, false, false, false, LATE_R>(
+  stage_body<Phys, NQ, EPW, C::NT, false, false, false, false, LATE_R>(
       lds, rhs, Q, nullptr, vgeo, sgeo, nullptr, e0, nreal, ntotal, vmapM, vmapP, bndy, 0.0, 0.0,
       0.0, p);
 }
@@ -1160,18 +1156,18 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_ker
 // facerhs! + updatesolution! of one stage in one pass (the volume term was
 // added to rhs by volume_kernel before): Qin -> Qout, rhs in place.
 template <class Phys, int NQ, int EPW>
-__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW, false>::NT)) void face_update_kernel(
+__global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT)) void face_update_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ vgeo, const double* __restrict__ sgeo, int64_t nreal,
     int64_t ntotal, const int64_t* __restrict__ vmapM, const int64_t* __restrict__ vmapP,
     const int64_t* __restrict__ bndy, double rka, double rkb, double dt,
     BlockOrder order, PhysParams p, int advection) {
-  using C = FusedCfg<Phys, NQ, EPW, false>;
+  using C = FusedCfg<Phys, NQ, EPW>;
   __shared__ __attribute__((aligned(16))) char lds[C::LDS];
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, 1, true, false>(lds, rhs, Qin, Qout, vgeo, sgeo, nullptr, e0,
+  stage_body<Phys, NQ, EPW, C::NT, false>(lds, rhs, Qin, Qout, vgeo, sgeo, nullptr, e0,
                                                    nreal, ntotal, vmapM, vmapP, bndy, rka, rkb,
                                                    dt, p, advection);
 }

@@ -124,14 +124,9 @@ inline bool one_wave_blocks(int64_t nreal, int small, int epw) {
 template <class Phys, int NQ, int EPW, bool MFMA = false>
 void launch_stage(const KArgs& a) {
   const int64_t nb = (a.nreal + EPW - 1) / EPW;
-  // measured on 3D N=4 (32^3): one prefetched face item per thread, the
-  // nodal pressure cached in LDS, workgroup sized by the volume nodes
-  constexpr bool WIDE = false;
-  constexpr int PF = 1;
-  constexpr bool PM_LDS = true;
-  constexpr int NT = FusedCfg<Phys, NQ, EPW, WIDE>::NT;
+  constexpr int NT = FusedCfg<Phys, NQ, EPW>::NT;
   const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
-  stage_kernel<Phys, NQ, EPW, WIDE, PF, PM_LDS, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
+  stage_kernel<Phys, NQ, EPW, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.D, a.nreal, a.ntotal, a.vmapM, a.vmapP, a.bndy, a.rka, a.rkb,
       a.dt, order, a.phys, a.advection);
@@ -167,10 +162,9 @@ constexpr int64_t kLargePrepNodes = 2000000;
 template <class Phys, int NQ, int EPW, bool MFMA = false>
 void launch_stage_prep(const KArgs& a) {
   const int64_t nb = (a.nreal + EPW - 1) / EPW;
-  constexpr int PF = 1;  // as launch_stage
-  constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
+  constexpr int NT = FusedCfg<Phys, NQ, EPW>::NT;
   const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
-  stage_prep_kernel<Phys, NQ, EPW, PF, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
+  stage_prep_kernel<Phys, NQ, EPW, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.pface, a.D, a.nreal, a.ntotal, a.rka, a.rkb, a.dt, order,
       a.phys, a.advection);
@@ -213,13 +207,13 @@ void launch_volume(int64_t nb, const KArgs& a) {
 // 287; N=7 8^3 (512 of 512) 177 / 177 and 152 / 153, 11^3 376 / 357 and 336 / 318.
 template <class Phys, int NQ, int EPW>
 bool late_rhs_pays(int64_t nb) {
-  constexpr int64_t fit = 256 * (160 * 1024 / FusedCfg<Phys, NQ, EPW, false>::LDS);
+  constexpr int64_t fit = 256 * (160 * 1024 / FusedCfg<Phys, NQ, EPW>::LDS);
   return nb > fit;
 }
 
 template <class Phys, int NQ, int EPW, bool LATE_R>
 void launch_face_form(int64_t nb, const KArgs& a) {
-  constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
+  constexpr int NT = FusedCfg<Phys, NQ, EPW>::NT;
   const BlockOrder order = inplace_order<Phys, NQ>(nb, a);
   face_kernel<Phys, NQ, EPW, LATE_R><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (const double*)a.vgeo, (const double*)a.sgeo, a.nreal,
@@ -248,7 +242,7 @@ int launch_update(const KArgs& a) {
 
 template <class Phys, int NQ, int EPW>
 void launch_face_update(int64_t nb, const KArgs& a) {
-  constexpr int NT = FusedCfg<Phys, NQ, EPW, false>::NT;
+  constexpr int NT = FusedCfg<Phys, NQ, EPW>::NT;
   const BlockOrder order = inplace_order<Phys, NQ>(nb, a, true);
   face_update_kernel<Phys, NQ, EPW><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
