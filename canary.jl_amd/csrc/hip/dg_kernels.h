@@ -760,9 +760,10 @@ constexpr bool late_rhs() {
 // opt-in facerhs_update, after a separate volumerhs); vgeo is then read for
 // MJI alone and D is not read.  UPDATE = false (with VOLUME = false) is
 // facerhs! alone: rhs -= face terms, Q untouched, neither vgeo nor Qout read;
-// LATE_R: rhs read after the face terms (late_rhs).
+// LATE_R: rhs read after the face terms (late_rhs).  EARLY: gathers before the
+// volume fluxes whatever gather_late says.
 template <class Phys, int NQ, int EPW, int NT, bool VOLUME = true, bool UPDATE = true,
-          bool PREP = false, bool MFMA = false, bool LATE_R = false>
+          bool PREP = false, bool MFMA = false, bool LATE_R = false, bool EARLY = false>
 __device__ __forceinline__ void stage_body(
     char* __restrict__ lds, typename Phys::Real* __restrict__ rhs,
     const typename Phys::Real* __restrict__ Qin, typename Phys::Real* __restrict__ Qout,
@@ -787,7 +788,7 @@ __device__ __forceinline__ void stage_body(
   // registers.  The code over them stays loops of one: written straight out, the
   // compiler moves the item's loads under `if (fval)` (10 x 10 loop 231.7 -> 235.4 us).
   constexpr int KP = 1;
-  constexpr bool LATE = VOLUME && gather_late<Phys, NQ>();
+  constexpr bool LATE = VOLUME && gather_late<Phys, NQ>() && !EARLY;
   constexpr bool N6 = stage_waves<Phys, NQ>() > 1;
   constexpr bool MAPS_LATE = LATE && !PREP && N6;
   constexpr bool STAGE_R = (!VOLUME && !LATE_R) || (VOLUME && N6);  // rhs waits in LDS for the face terms
@@ -1115,7 +1116,7 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, N
 
 // The fused stage over the prepared arrays (see Prepared): the same
 // arithmetic and order, fewer bytes.
-template <class Phys, int NQ, int EPW, bool MFMA = false>
+template <class Phys, int NQ, int EPW, bool MFMA = false, bool EARLY = false>
 __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>())) void stage_prep_kernel(
     double* __restrict__ rhs, const double* __restrict__ Qin, double* __restrict__ Qout,
     const double* __restrict__ pvgeo, const double* __restrict__ psgeo,
@@ -1127,7 +1128,7 @@ __global__ __launch_bounds__((FusedCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, N
   const int64_t blk = stage_block(blockIdx.x, order);
   const int64_t e0 = blk * EPW;
   if (e0 >= nreal) return;  // whole workgroup leaves together
-  stage_body<Phys, NQ, EPW, C::NT, true, true, true, MFMA>(
+  stage_body<Phys, NQ, EPW, C::NT, true, true, true, MFMA, false, EARLY>(
       lds, rhs, Qin, Qout, pvgeo, psgeo, D, e0, nreal, ntotal, nullptr,
       reinterpret_cast<const int64_t*>(pface), nullptr, rka, rkb, dt, p, advection);
 }

@@ -159,12 +159,23 @@ constexpr int large_prep_epw() {
 }
 constexpr int64_t kLargePrepNodes = 2000000;
 
-template <class Phys, int NQ, int EPW, bool MFMA = false>
+// The exact-order prepared 3D stage below N = 6 gathers early (see gather_late)
+// on a mesh of at most one wave a SIMD: there no other wave covers the gather's
+// latency, and its registers limit nothing.  us for two steps, late / early: N=1 8^3
+// 95 / 87, 14^3 105 / 97, 20^3 (1,000 waves) 175 / 168, 27^3 176 / 180; N=2 9^3 90 / 83, 18^3 175 / 179;
+// N=3 7^3 87 / 82, 10^3 103 / 98, 13^3 145 / 147; N=4 8^3 114 / 112, 11^3 164 / 167; N=5 5^3 86 / 84, 7^3
+// 115 / 117.  (Over the reference arrays the late gathers are level or ahead there too.)
+template <class Phys, int NQ, int EPW>
+bool gather_early(int64_t nreal) {
+  return (nreal + EPW - 1) / EPW * (FusedCfg<Phys, NQ, EPW>::NT / 64) <= 4 * 256;
+}
+
+template <class Phys, int NQ, int EPW, bool MFMA = false, bool EARLY = false>
 void launch_stage_prep(const KArgs& a) {
   const int64_t nb = (a.nreal + EPW - 1) / EPW;
   constexpr int NT = FusedCfg<Phys, NQ, EPW>::NT;
   const BlockOrder order = block_order(nb, walk_back(a.Q, a.Qout));
-  stage_prep_kernel<Phys, NQ, EPW, MFMA><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
+  stage_prep_kernel<Phys, NQ, EPW, MFMA, EARLY><<<dim3((unsigned)(8 * order.chunk)), dim3(NT), 0, a.stream>>>(
       (double*)a.rhs, (const double*)a.Q, (double*)a.Qout, (const double*)a.vgeo,
       (const double*)a.sgeo, a.pface, a.D, a.nreal, a.ntotal, a.rka, a.rkb, a.dt, order,
       a.phys, a.advection);
@@ -183,6 +194,9 @@ void launch_stage_prep_if(const KArgs& a) {
     if constexpr (BIG > EPW)
       if (a.nreal * Shape<Phys, NQ>::Np >= kLargePrepNodes)
         return launch_stage_prep<Phys, NQ, BIG, MFMA>(a);
+    if constexpr (Phys::DIM == 3 && gather_late<Phys, NQ>() && NQ < 7)
+      if (gather_early<Phys, NQ, EPW>(a.nreal))
+        return launch_stage_prep<Phys, NQ, EPW, MFMA, true>(a);
     launch_stage_prep<Phys, NQ, EPW, MFMA>(a);
   }
 }
