@@ -680,7 +680,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
-                     "kernel": "stage_prep_kernel<Euler3DFma,5,1,1,false> (fused volume+face+update "
+                     "kernel": "stage_prep_kernel<Euler3DFma,5,1,false,false> (fused volume+face+update "
                                "over the prepared arrays)",
                      "bytes_per_element_stage": algorithmic_bytes(3, s.N),
                      "bytes_per_element_stage_own": own_bytes,
@@ -1179,7 +1179,7 @@ def served_form(nreq, rate, seed=2024, graph=False):
                                     "median": float("%.3e" % float(np.median(errs)))}}
 
 
-HEADLINE_KERNEL = "stage_prep_kernel<canary::Euler3DFma, 5, 1, 1, false>"
+HEADLINE_KERNEL = "stage_prep_kernel<canary::Euler3DFma, 5, 1, false, false>"
 
 
 def _csv_rows(d, pattern):
