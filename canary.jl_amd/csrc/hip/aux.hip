@@ -38,8 +38,10 @@ __device__ __forceinline__ void aux_error(unsigned long long code, long long a, 
 }
 
 constexpr int RED_BLOCKS = CANARY_REDUCE_WORK;
-// 512 lanes: four workgroups a CU, 32 waves, so enough loads are in flight
-// with one node per lane and turn.
+// 512 lanes, 1,024 workgroups: enough loads are in flight with one node per lane
+// and turn.  All are resident at once (four a CU, 32 waves) in the energy and the
+// shallow-water cfl kernels; the Euler cfl (74-76 VGPRs) and Courant kernels (72)
+// fit three a CU, so a quarter of their workgroups runs in a second round.
 constexpr int RED_THREADS = 512;
 constexpr int RED_STRIDE = RED_BLOCKS * RED_THREADS;
 
@@ -48,7 +50,7 @@ constexpr int RED_STRIDE = RED_BLOCKS * RED_THREADS;
 // is 1,024 far-apart fronts), with (element, node) carried along instead of
 // divided out per node (a 64-bit division by a runtime Np is some 100
 // instructions).  us per call at 32^3 N=4 (both kernels), before -> after:
-// energy 53 -> 32, cfl 89 -> 82 (459 MB: 5.8 TB/s), courant 76 -> 62.
+// energy 53 -> 32, cfl 89 -> 82 (459 MB: 5.6 TB/s), courant 76 -> 62.
 struct Walk {
   int64_t e, n, Np;
   int de, dn;

@@ -119,7 +119,7 @@ __global__ __launch_bounds__((BCfg<Phys, NQ, EPW>::NT), (stage_waves<Phys, NQ>()
   // one face item prefetched and five waves a SIMD at 3D N=6, as the
   // single-solve stage.  Six N=6 bubbles of 8^3..13^3, us a step, no item
   // prefetched against this: exact 1,129 / 960, contracted 903 / 775; prepared
-  // 1,036 / 980 and 820 / 743
+  // 1,036 / 980 (the one that spills, 16 bytes a lane) and 820 / 743
   solve_stage<Phys, NQ, EPW, C::NT, PREP>(lds, sv, it.e0, parity, rka, rkb, p);
 }
 

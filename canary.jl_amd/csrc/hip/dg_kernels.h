@@ -508,7 +508,9 @@ __device__ __forceinline__ void face_terms_at_node(Real* r, const Real* sC, cons
 // until r is stored), and the node owner takes one term per pair, in
 // ascending order.  Where two items of a pair name one node, which no
 // numbering of a face does, the owners look through all items instead, which
-// is right for every map and several times the work.
+// is right for every map and several times the work.  Bound by its barriers and
+// LDS round trips, little beside the rest of a launch: facerhs! at 3D N=7 16^3, us,
+// canonical map 70, every face reversed 71 (searched 285); N=4 25^3 83 and 86 (183).
 template <int DIM, int NQ, int EPW, int NT, int NSR, int BUF, int TSTR, class Real, class VidT>
 __device__ __forceinline__ void face_terms_any_map(Real* r, const Real* sB, const VidT* sV,
                                                    Real* tab, int* sFlag, VidT novid, int nv,
@@ -722,7 +724,8 @@ struct FusedCfg {
 // exact-order 3D kernels (32^3 N=4, reference arrays: 1,422 -> 1,377 us a step;
 // N=7: 1,342 -> 1,235) and the contracted ones from N = 6 on; the contracted
 // ones below are faster early (N=5: 1,042 against 1,058), as is 2D (10 x 10
-// meshes wait for latency alone: 240 against 269 us for 50 stages).
+// meshes wait for latency alone: 240 against 269 us for 50 stages), and as the
+// exact prepared stage is on a mesh of one wave a SIMD (gather_early, launch.h).
 //
 // 3D N = 6 has 343 nodes in six waves: at 96 VGPRs five waves fit a SIMD and
 // three workgroups a CU, above that two.  It is built for that (stage_waves),

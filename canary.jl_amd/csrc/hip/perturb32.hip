@@ -63,8 +63,8 @@ __device__ __forceinline__ void p32_error(unsigned long long code, long long fac
 // The stage was bound by VALU issue (0.9 of the cycles at 3D N=4 48^3: 1,098
 // instructions a wave, a third of them the library's log1p and expm1 and
 // IEEE divisions and roots).  The series and the refined hardware estimates
-// below take them to about 700 and leave it bound by memory: 2,265 -> 2,065 us
-// a step with the block order of dg_kernels.h, 1,974 with single_epw's blocks
+// below take them to about 700 and leave it bound by memory: 2,251 -> 2,065 us
+// a step with the block order of dg_kernels.h, 1,970 with single_epw's blocks
 // (10.5 GB of least traffic, 5.3 TB/s).  Relative L2 error of one stage's
 // register against 64 bits, before -> after: ru 7.3e-8 the same, rv 7.1e-7 ->
 // 5.7e-7, rw 7.3e-7 -> 6.0e-7, rho and rho*theta the same.

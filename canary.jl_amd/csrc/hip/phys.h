@@ -486,10 +486,10 @@ struct SWE2DFma : SWE2D {
 // unit is built without contraction), so each launch form gives the same
 // bits.  b = still depth is read only and h is already the deviation from
 // it, so FP32 keeps h's relative precision.  The kernels issued vector
-// instructions in 0.85 of the cycles (777 of them at N=4, a third IEEE
-// divisions and roots; now 604): 64 solves per step 398 -> 390 us over the
-// reference arrays, 48 solves prepared in one launch 226 -> 212.  One stage's
-// register against 64 bits: h 8% closer, the momenta the same on average.
+// instructions in 0.85 of the cycles, a third of them IEEE divisions and
+// roots: a step of 64 solves over the reference arrays, a kernel per order, 405 ->
+// 400 us, of 21 small ones in one launch 103 -> 98, prepared 91 -> 86.
+// Error against 64 bits over 72 ensembles: 1.000 of the IEEE form's.
 struct SWE2DF32 {
   using Real = float;
   static constexpr bool EXACT = false;
