@@ -23,11 +23,11 @@ _NSG = {3: 5, 2: 4}
 
 
 # The host side of a call is a few dozen checks and one foreign call; calls on
-# small meshes are issued no faster than it runs, so it is kept short (of a
-# rank's pack, unpack and stage it hides nearly all: 43.8 -> 43.4 us).  Pointers
-# go over as integers (the argument types are void pointers), the current
-# stream is read as a raw handle, and a tensor that passes is checked in one
-# expression.
+# small meshes are issued no faster than it runs, so it is kept short (where the
+# GPU is slower it gains little: a rank's pack, unpack and stage 43.8 -> 43.4 us).
+# Pointers go over as integers (the argument types are void pointers), the
+# current stream is read as a raw handle, and a tensor that passes is checked
+# in one expression.
 def _ptr(t):
     return t.data_ptr()
 
