@@ -139,15 +139,34 @@ __device__ __attribute__((noinline)) float expm1_klog1p(float a, float b, float 
   return expm1f(kappa * log1pf(a / b));
 }
 
-// (the estimated quotient is not finite where it does not hold: a background
-// above 2^126, where it would be zero, has an infinite P0)
-__device__ __forceinline__ float pprime(float P0, float rt0, float rtp, const P32Params& p) {
-  const float x = div_est(rtp, rt0, __builtin_amdgcn_rcpf(rt0));
-  if (!(fabsf(x) <= p.xmax)) return P0 * expm1_klog1p(rtp, rt0, p.kappa);
+// The series in x = rtp / rt0, whose estimate is not finite where it does not
+// hold (a background above 2^126, where it would be zero, has an infinite P0).
+__device__ __forceinline__ float series_x(float rt0, float rtp) {
+  return div_est(rtp, rt0, __builtin_amdgcn_rcpf(rt0));
+}
+__device__ __forceinline__ float series_sum(float x, const P32Params& p) {
   float a = p.c[kSeries - 1];
 #pragma unroll
   for (int i = kSeries - 2; i >= 0; --i) a = fmaf(a, x, p.c[i]);
-  return P0 * (x * a);
+  return x * a;
+}
+
+__device__ __forceinline__ float pprime(float P0, float rt0, float rtp, const P32Params& p) {
+  const float x = series_x(rt0, rtp);
+  if (!(fabsf(x) <= p.xmax)) return P0 * expm1_klog1p(rtp, rt0, p.kappa);
+  return P0 * series_sum(x, p);
+}
+
+// P' and 1 / rho of a node, both estimates tested in one branch.
+__device__ __forceinline__ void node_state(float P0, float rt0, float rtp, float rho,
+                                           const P32Params& p, float& Pp, float& ri) {
+  const float x = series_x(rt0, rtp);
+  ri = recip_est(rho);
+  Pp = P0 * series_sum(x, p);
+  if (!((fabsf(x) <= p.xmax) & recip_ok(ri))) {
+    Pp = P0 * expm1_klog1p(rtp, rt0, p.kappa);
+    ri = 1.f / rho;
+  }
 }
 
 // ------------------------------------------------------------ prepare
@@ -366,15 +385,15 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
   if (t < NQ * NQ) L.D[t] = (float)dval;
   if (valid) {
     const float rho0 = b0, rt0 = b1, P0 = b2;
-    const float Pp = pprime(P0, rt0, q[E], p);
+    const float rho = rho0 + q[RHO], rt = rt0 + q[E];
+    float Pp, ri;
+    node_state(P0, rt0, q[E], rho, p, Pp, ri);
 #pragma unroll
     for (int s = 0; s < NS; ++s) L.Q[slot][s * Np + n] = q[s];
     L.Bg[slot][n] = rho0;
     L.Bg[slot][Np + n] = rt0;
     L.Bg[slot][2 * Np + n] = P0;
     L.Bg[slot][3 * Np + n] = Pp;
-    const float rho = rho0 + q[RHO], rt = rt0 + q[E];
-    const float ri = recip32(rho);
     // physical perturbation fluxes f[c][s] along coordinate c
     float f[DIM][NS];
 #pragma unroll
@@ -487,9 +506,8 @@ __device__ __forceinline__ void body(Lds32<DIM, NQ, EPW>& L, RT* __restrict__ rh
   // The node owner takes its own face terms, in ascending face order, and
   // updates; its results go to LDS and from there out in storage order.
   if (valid) {
-    // the reference's MJI is 1 ./ MJ; the estimate holds where it is a normal number
-    double MJI = FastOps::recip((double)MJg);
-    if (__builtin_expect(!__builtin_amdgcn_class(MJI, 0x108), 0)) MJI = 1.0 / (double)MJg;
+    // the reference's MJI is 1 ./ MJ (zero and infinity as IEEE division has them)
+    const double MJI = __builtin_amdgcn_div_fixup(FastOps::recip((double)MJg), (double)MJg, 1.0);
     const int ni = n % NQ, nj = (n / NQ) % NQ, nk = DIM == 3 ? n / (NQ * NQ) : 0;
     const float* fc = L.B[slot];
 #pragma unroll

@@ -106,3 +106,21 @@ def test_precision_form(cuda, dim, N, what, form):
     assert not np.isfinite(r[face_nodes(dim, N), dim, 0]).any()
     # nothing reaches the elements that do not touch it
     assert np.isfinite(r[~face_nodes(dim, N), dim, :][:, 1:]).all()
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_node_without_volume(cuda, mixed):
+    """MJ = 0 at a node (MJI infinite): the update is infinite there, not NaN."""
+    s = small_setup(0, 2, 3, Ne=2, periodic=(True, True), gravity=0.0)
+    s.vgeo = np.array(s.vgeo, order="F", copy=True)
+    n = 5  # inside the element: no face term
+    s.vgeo[n, 4, 0], s.vgeo[n, 5, 0] = 0.0, np.inf
+    Q0 = P.uniform_rest_state(s, 1.25, 1e5)
+    q = np.zeros(Q0.shape, order="F")
+    q[:, :2, :] = np.random.default_rng(0).uniform(1.0, 2.0, size=q[:, :2, :].shape)
+    pf = Perturb32(s, Q0, np.asfortranarray(Q0 + q), mixed=mixed)
+    pf.stage(1.0, 0.5, 1e-3)
+    pf.check()
+    got = host(pf.q, Q0.shape)
+    assert np.isinf(got[n, :2, 0]).all()
+    assert np.isfinite(np.delete(got[:, :, 0], n, axis=0)).all() and np.isfinite(got[:, :, 1:]).all()
